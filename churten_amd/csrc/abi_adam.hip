@@ -91,7 +91,7 @@ int ts_adam_step_noalloc(const ts_rt_buf* bufs, ts_dtype dtype, void* state_step
   if (err != 0) return err;
   const auto c = make_call(bufs, state_steps, {lr, beta1, beta2, eps, weight_decay},
                            active_mask, R, T, flags, out_zero, stream, ws,
-                           sizeof(double) * churten::kPreStride * churten::kScratchReplicas);
+                           ts_workspace_bytes(R));
   return churten::adam_run<false>(dtype, c, nullptr, 0);
 }
 

@@ -71,6 +71,8 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <initializer_list>
 #include <type_traits>
 
@@ -235,6 +237,21 @@ struct Operands {
   int64_t stride_t[kMaxOperands];
 };
 
+// A call that runs as a single launch ("One launch per call", below): `nonce`
+// identifies it (0: not such a call), `entries` are its records of kEntryWords
+// words, one per replica, `steps` is the counter its heads advance where `bump`
+// says so, `out_zero` the result they clear, and workgroups before `early`
+// start before the heads are done.
+template <typename T>
+struct Single {
+  uint64_t nonce;
+  uint64_t* entries;
+  T* steps;
+  T* out_zero;
+  uint32_t early;
+  bool bump;
+};
+
 // (R,) inputs: the step counter, up to five hyperparameter vectors and the mask.
 // `pre`: the call's per-replica constants (kPreWords doubles per replica,
 // replica r at pre + kPreStride * r), written by the preparation launch; null
@@ -248,6 +265,7 @@ struct Vectors {
   const uint8_t* mask;
   const double* pre;
   uint32_t ilp_rows;
+  Single<T> one;
 };
 
 // Whether row r takes the vector path of torch's fused optimizer kernels (and
@@ -344,9 +362,29 @@ __device__ __forceinline__ void stream_tile_of_block(const Grid& g, uint32_t& r,
   t0 = int64_t(m - r * g.tiles_per_row + 1) * TILE;
 }
 
+// Replica r's hyperparameter. No kernel writes these vectors, so they are read
+// as constants: with a workgroup's one r that is a scalar load whatever the
+// kernel stores elsewhere. A 16-bit value comes out of the aligned dword that
+// holds it (which never leaves the value's page; there is no 16-bit scalar
+// load).
 template <typename T>
 __device__ __forceinline__ double hyper_at(const T* h, uint32_t r) {
-  return static_cast<double>(widen(h[r]));
+  if constexpr (sizeof(T) == 2) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(h + r);
+    const auto* word =
+        reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(at & ~uintptr_t(3));
+    const uint16_t bits = static_cast<uint16_t>(*word >> (8 * (at & 2)));
+    return static_cast<double>(widen(__builtin_bit_cast(T, bits)));
+  } else {
+    return static_cast<double>(*reinterpret_cast<const __attribute__((address_space(4))) T*>(
+        reinterpret_cast<uintptr_t>(h + r)));
+  }
+}
+
+// Replica r's step. Not a constant: a single launch's heads store it.
+template <typename T>
+__device__ __forceinline__ double step_at(const T* steps, uint32_t r) {
+  return static_cast<double>(widen(steps[r]));
 }
 
 // Lane `lane`'s x, for every lane of the wavefront (that lane must be active).
@@ -466,15 +504,18 @@ constexpr int stream_unroll(int fp32, int bf16_state, int narrow, int wide) {
 // parameters stay in float32 (the state is widened on load and rounded to
 // nearest-even on store).
 //
-// Per-replica constants. `prologue<false>` derives a replica's constants in
-// every workgroup (Adam: two fp64 pow and the step size's divide; Adagrad: an
-// fp64 divide); `prologue<true>` reads them from the call's workspace, where
-// the preparation launch (`precompute`, once per replica and call, after the
-// step bump) put them. Both give the same bits: the workspace holds the
-// math-type values widened to double (Adam's divisor of sqrt(v) is a double
-// already). kPreWords is the number of such doubles (0: nothing worth
-// hoisting, the policy never reads a workspace). `reads_state` is decided from
-// the (R,) vectors alone, so the drivers issue their loads before the prologue.
+// Per-replica constants. `derive` computes a replica's from its bumped step
+// (Adam: two fp64 pow and the step size's divide; Adagrad: an fp64 divide; SGD:
+// whether it is a first step); `hypers` and `set` read the hyperparameters and
+// take the constants (kConstants doubles, as `constants` gives them) from the
+// call's workspace, where the preparation launch or a single launch's heads put
+// them. Both give the same bits: the workspace holds the math-type values
+// widened to double (Adam's divisor of sqrt(v) is a double already). kPreWords
+// is the number of doubles that are worth a preparation launch (0: the policy's
+// two-launch calls never read a workspace). `reads_state` is decided from the
+// (R,) vectors alone, so the drivers issue their loads before the constants;
+// `may_read_state` and `needs_entry` are its like in a single launch, where the
+// step may be seen from before or after the bump.
 // `decays` / `drop_decay`: whether the replica's weight-decay term is live, and
 // a copy of its constants with the decay set to a literal zero (the element
 // math then skips the term, exactly as it does for a zero decay at run time).
@@ -546,7 +587,7 @@ constexpr int stream_unroll(int fp32, int bf16_state, int narrow, int wide) {
 // the scalar one).
 
 // Without a workspace, float32 Adam derives its constants once per wavefront
-// (wave_prologue: the two pow and two divides spread over even and odd lanes,
+// (wave_derive: the two pow and two divides spread over even and odd lanes,
 // 280 VALU instructions per workgroup instead of 425), and with it amsgrad
 // moved to one pack per thread. Same-process A/B against the per-lane form
 // (3 rounds, one box): config 1 +22%, config 2 +8.9%, config-5 buffers +2.5%,
@@ -634,40 +675,37 @@ struct AdamPolicy {
     AdamHyper h;
     AdamConsts<M> c;
   };
+  static constexpr int kConstants = 2;
   // The step size and sqrt(v)'s divisor of the bumped step (adam_consts).
-  __device__ static AdamConsts<M> consts(const Vectors<T>& v, uint32_t r) {
+  __device__ static AdamConsts<M> consts(const Vectors<T>& v, uint32_t r, double step) {
     M bc1, bc2s;
-    adam_bias_corrections<M>(hyper_at(v.h[1], r), hyper_at(v.h[2], r), hyper_at(v.steps, r),
-                             bc1, bc2s);
+    adam_bias_corrections<M>(hyper_at(v.h[1], r), hyper_at(v.h[2], r), step, bc1, bc2s);
     return adam_consts<M>(hyper_at(v.h[0], r), bc1, bc2s);
   }
-  __device__ static void precompute(const Vectors<T>& v, uint32_t r, double* out) {
-    const AdamConsts<M> c = consts(v, r);
-    out[0] = static_cast<double>(c.step_size);
-    out[1] = c.bc2s_div;
-  }
-  template <bool PRE>
-  __device__ static void prologue(const Vectors<T>& v, uint32_t r, Rep& rep) {
+  __device__ static void derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
     hypers(v, r, rep);
-    if constexpr (PRE) {
-      rep.c.step_size = static_cast<M>(v.pre[kPreStride * r]);
-      rep.c.bc2s_div = v.pre[kPreStride * r + 1];
-    } else {
-      rep.c = consts(v, r);
-    }
+    rep.c = consts(v, r, step);
   }
-  // prologue<false> for a replica that every lane of the wavefront shares.
+  __device__ static void constants(const Rep& rep, double* out) {
+    out[0] = static_cast<double>(rep.c.step_size);
+    out[1] = rep.c.bc2s_div;
+  }
+  __device__ static void set(const double* w, Rep& rep) {
+    rep.c.step_size = static_cast<M>(w[0]);
+    rep.c.bc2s_div = w[1];
+  }
+  // derive() for a replica that every lane of the wavefront shares.
   // The two bias corrections' pow run as one, beta1's on even lanes and
   // beta2's on odd ones, and so do the step size's divide and (float math)
   // the divide that gives sqrt(v)'s divisor; lanes 0 and 1 then hand their
   // values to the whole wavefront. Each value comes from the same operations
   // on the same operands as in consts(), so the bits are the same, at about
   // half of consts()'s fp64 instructions.
-  __device__ static void wave_prologue(const Vectors<T>& v, uint32_t r, Rep& rep) {
+  __device__ static void wave_derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
     hypers(v, r, rep);
     const bool odd = (__lane_id() & 1) != 0;
     const double bc = adam_bias_correction(odd ? rep.h.beta2 : rep.h.beta1,
-                                           static_cast<float>(hyper_at(v.steps, r)));
+                                           static_cast<float>(step));
     if constexpr (std::is_same<M, float>::value) {
       // Even lanes: lr / bias_correction1; odd lanes: 1 / bias_correction2_sqrt,
       // each correction narrowed to float first (adam_consts).
@@ -689,6 +727,8 @@ struct AdamPolicy {
     rep.h.weight_decay = hyper_at(v.h[4], r);
   }
   __device__ static bool reads_state(const Vectors<T>&, uint32_t) { return true; }
+  __device__ static bool may_read_state(T, bool) { return true; }
+  __device__ static bool needs_entry(T, bool) { return true; }
   __device__ static bool decays(const Rep& rep) { return rep.h.weight_decay != 0; }
   __device__ static void drop_decay(Rep& rep) { rep.h.weight_decay = 0.0; }
   __device__ static void update(M& p, M g, M (&s)[NS], const Rep& rep, bool maximize) {
@@ -763,20 +803,30 @@ struct SgdPolicy {
     SgdHyper<double> h;
     bool first;
   };
-  __device__ static void precompute(const Vectors<T>&, uint32_t, double*) {}
-  template <bool PRE>
-  __device__ static void prologue(const Vectors<T>& v, uint32_t r, Rep& rep) {
+  static constexpr int kConstants = 1;
+  __device__ static void hypers(const Vectors<T>& v, uint32_t r, Rep& rep) {
     rep.h.lr = hyper_at(v.h[0], r);
     rep.h.momentum = hyper_at(v.h[1], r);
     rep.h.dampening = hyper_at(v.h[2], r);
     rep.h.weight_decay = hyper_at(v.h[3], r);
-    rep.first = widen(v.steps[r]) == M(1);
   }
+  // The constant: 1 on the replica's first step, else 0.
+  __device__ static void derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
+    hypers(v, r, rep);
+    rep.first = step == 1.0;
+  }
+  __device__ static void constants(const Rep& rep, double* out) { out[0] = rep.first ? 1.0 : 0.0; }
+  __device__ static void set(const double* w, Rep& rep) { rep.first = w[0] != 0.0; }
   // On a replica's first step the buffer is overwritten by the gradient
   // without being read, so it is not fetched.
   __device__ static bool reads_state(const Vectors<T>& v, uint32_t r) {
     return widen(v.steps[r]) != M(1);
   }
+  // The same from a step read while it may be bumped: 0 is from before a first
+  // step's bump, and only 1 needs the entry (a first step's new step, or the
+  // old one of the second).
+  __device__ static bool may_read_state(T x, bool bump) { return widen(x) != M(bump ? 0 : 1); }
+  __device__ static bool needs_entry(T x, bool bump) { return bump && widen(x) == M(1); }
   __device__ static bool decays(const Rep& rep) { return rep.h.weight_decay != 0; }
   __device__ static void drop_decay(Rep& rep) { rep.h.weight_decay = 0.0; }
   __device__ static void update(M& p, M g, M (&s)[NS > 0 ? NS : 1], const Rep& rep,
@@ -837,24 +887,23 @@ struct AdagradPolicy {
     AdagradHyper h;
     bool once;  // float16 state sum rounded once (ilp_row)
   };
-  // corrected_lr of the bumped step.
-  __device__ static void precompute(const Vectors<T>& v, uint32_t r, double* out) {
-    out[0] = adagrad_corrected_lr(hyper_at(v.h[0], r), hyper_at(v.h[1], r),
-                                  static_cast<float>(widen(v.steps[r])));
+  static constexpr int kConstants = 1;
+  // The constant is corrected_lr of the bumped step.
+  __device__ static void derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
+    hypers(v, r, rep);
+    rep.h.corrected_lr = adagrad_corrected_lr(hyper_at(v.h[0], r), hyper_at(v.h[1], r),
+                                              static_cast<float>(step));
   }
-  template <bool PRE>
-  __device__ static void prologue(const Vectors<T>& v, uint32_t r, Rep& rep) {
+  __device__ static void constants(const Rep& rep, double* out) { out[0] = rep.h.corrected_lr; }
+  __device__ static void set(const double* w, Rep& rep) { rep.h.corrected_lr = w[0]; }
+  __device__ static void hypers(const Vectors<T>& v, uint32_t r, Rep& rep) {
     rep.h.weight_decay = hyper_at(v.h[2], r);
     rep.h.eps = hyper_at(v.h[3], r);
     rep.once = kVariant && ilp_row(v.ilp_rows, r);
-    if constexpr (PRE) {
-      rep.h.corrected_lr = v.pre[kPreStride * r];
-    } else {
-      rep.h.corrected_lr = adagrad_corrected_lr(hyper_at(v.h[0], r), hyper_at(v.h[1], r),
-                                                static_cast<float>(widen(v.steps[r])));
-    }
   }
   __device__ static bool reads_state(const Vectors<T>&, uint32_t) { return true; }
+  __device__ static bool may_read_state(T, bool) { return true; }
+  __device__ static bool needs_entry(T, bool) { return true; }
   __device__ static bool decays(const Rep& rep) { return rep.h.weight_decay != 0; }
   __device__ static void drop_decay(Rep& rep) { rep.h.weight_decay = 0.0; }
   // float16 parameters and state. torch's fused Adagrad stores the state sum
@@ -954,24 +1003,27 @@ struct AdagradF32Policy {
   struct Rep {
     AdagradF32Hyper h;
   };
-  __device__ static void precompute(const Vectors<T>& v, uint32_t r, double* out) {
-    out[0] = static_cast<double>(
-        adagrad_corrected_lr_f32(hyper_at(v.h[0], r), hyper_at(v.h[1], r), hyper_at(v.steps, r)));
+  static constexpr int kConstants = 1;
+  __device__ static void derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
+    hypers(v, r, rep);
+    rep.h.corrected_lr =
+        adagrad_corrected_lr_f32(hyper_at(v.h[0], r), hyper_at(v.h[1], r), step);
   }
-  template <bool PRE>
-  __device__ static void prologue(const Vectors<T>& v, uint32_t r, Rep& rep) {
+  __device__ static void constants(const Rep& rep, double* out) {
+    out[0] = static_cast<double>(rep.h.corrected_lr);
+  }
+  __device__ static void set(const double* w, Rep& rep) {
+    rep.h.corrected_lr = static_cast<float>(w[0]);
+  }
+  __device__ static void hypers(const Vectors<T>& v, uint32_t r, Rep& rep) {
     const double wd = hyper_at(v.h[2], r);
     rep.h.weight_decay = static_cast<float>(wd);
     rep.h.has_weight_decay = wd != 0.0;
     rep.h.eps = static_cast<float>(hyper_at(v.h[3], r));
-    if constexpr (PRE) {
-      rep.h.corrected_lr = static_cast<float>(v.pre[kPreStride * r]);
-    } else {
-      rep.h.corrected_lr = adagrad_corrected_lr_f32(hyper_at(v.h[0], r), hyper_at(v.h[1], r),
-                                                    hyper_at(v.steps, r));
-    }
   }
   __device__ static bool reads_state(const Vectors<T>&, uint32_t) { return true; }
+  __device__ static bool may_read_state(T, bool) { return true; }
+  __device__ static bool needs_entry(T, bool) { return true; }
   __device__ static bool decays(const Rep& rep) { return rep.h.has_weight_decay; }
   __device__ static void drop_decay(Rep& rep) {
     rep.h.weight_decay = 0.0f;
@@ -1052,9 +1104,9 @@ constexpr bool stream_scalar_mask() {
 }
 
 // A policy's constants for a replica that a whole workgroup works on: its
-// `wave_prologue` (derived once per wavefront, the work spread over lanes)
-// where it sets kWavePrologue and the constants are derived, else
-// `prologue<PRE>`. Every lane of the wavefront must be active.
+// `wave_derive` (once per wavefront, the work spread over lanes) where it sets
+// kWavePrologue and the constants are derived, else `derive` or the workspace's.
+// Every lane of the wavefront must be active.
 template <typename P, typename = void>
 struct wave_prologue_of {
   static constexpr bool value = false;
@@ -1063,13 +1115,32 @@ template <typename P>
 struct wave_prologue_of<P, std::void_t<decltype(P::kWavePrologue)>> {
   static constexpr bool value = P::kWavePrologue;
 };
+template <typename P>
+__device__ __forceinline__ void uniform_derive(const Vectors<typename P::T>& v, uint32_t r,
+                                               double step, typename P::Rep& rep) {
+  if constexpr (wave_prologue_of<P>::value) {
+    P::wave_derive(v, r, step, rep);
+  } else {
+    P::derive(v, r, step, rep);
+  }
+}
+template <typename P, bool PRE>
+__device__ __forceinline__ void prologue(const Vectors<typename P::T>& v, uint32_t r,
+                                         typename P::Rep& rep) {
+  if constexpr (PRE) {
+    P::hypers(v, r, rep);
+    P::set(v.pre + kPreStride * r, rep);
+  } else {
+    P::derive(v, r, step_at(v.steps, r), rep);
+  }
+}
 template <typename P, bool PRE>
 __device__ __forceinline__ void uniform_prologue(const Vectors<typename P::T>& v, uint32_t r,
                                                  typename P::Rep& rep) {
-  if constexpr (!PRE && wave_prologue_of<P>::value) {
-    P::wave_prologue(v, r, rep);
+  if constexpr (PRE) {
+    prologue<P, true>(v, r, rep);
   } else {
-    P::template prologue<PRE>(v, r, rep);
+    uniform_derive<P>(v, r, step_at(v.steps, r), rep);
   }
 }
 
@@ -1129,6 +1200,216 @@ __device__ __forceinline__ bool mask_byte_scalar(const uint8_t* mask, uint32_t r
   const auto* word =
       reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(at & ~uintptr_t(3));
   return ((*word >> (8 * (at & 3))) & 0xFFu) != 0;
+}
+
+// ---------------------------------------------------------------------------
+// One launch per call
+// ---------------------------------------------------------------------------
+// A call's constants depend on the bumped step, and every replica's step is to
+// advance once. Two launches (preparation or bump, then update) order that by
+// themselves; the first costs 2-3.5 us per call, its own time and the gap
+// behind it (same-process A/B of the update with and without it: 4 x 4522 SGD
+// 7.4 -> 4.0 us, 8 x 265,484 Adam 14.6 -> 11.4, 100 x 265,484 Adam with amsgrad
+// 116.0 -> 113.0). A call with room for the entries below runs as one launch:
+//
+//   * The grid's first R workgroups are the replicas' heads. A head reads
+//     steps[r], computes the constants of the bumped step, writes them to the
+//     replica's entry in the workspace, and only when memory has them stores
+//     the bumped step.
+//   * Every other wavefront reads steps[r], and after that looks into the
+//     entry. If the constants are there, it takes them. If not, the step it
+//     read is the one from before the bump (the head stores the new one after
+//     the entry), and it computes the constants from that, the same operations
+//     on the same operands. Nothing ever waits for another workgroup.
+//
+// An entry holds kConstants doubles as 2 * kConstants 8-byte words, each half a
+// double next to a 32-bit tag of the launch: a word is this launch's or it is
+// not, whatever the memory held before and in whatever order the words arrive.
+// Tags do not repeat within 2^32 launches of a process (next_nonce). A call
+// that is being captured into a graph, whose replays would repeat them, takes
+// two launches.
+//
+// The look goes through the scalar cache where it can: as a vector load it
+// cost large launches 2% (it queues behind the streaming loads, like a vector
+// read of the mask). A miss there means a second look, at memory itself, since
+// the line may have been cached before the head wrote it. The first workgroups
+// of a dense launch (`early`: those that start before the heads can be done)
+// look at memory only, and compute the constants meanwhile, while their data is
+// on the way: 64 x 545,100 Adagrad and 100 x 265,484 amsgrad ran 1% faster so
+// than with the scalar look first. Segmented launches lost with it (5 x 4795
+// Adam 7%, 16 x 3.15M 1%).
+//
+// Same-process A/B of whole calls against two launches: 4 x 4522 SGD 1.7x,
+// 8 x 265,484 Adam 1.22x, 32 x 265,484 segmented Adam 1.07x (with its loads
+// issued before the constants), 100 x 265,484 amsgrad +2.1%, 64 x 545,100
+// Adagrad +1.5%, 32 x 545,100 segmented SGD +3%, 16 x 25.2M Adam +0.4%,
+// 100 x 545,100 bfloat16 Adam -0.4% to 0 (24 rows: +1.7%).
+constexpr int64_t kEntryWords = 16;  // 8-byte words per replica: a 128-byte line
+constexpr uint32_t kEarlyBlocks = 4096;
+constexpr int64_t kSingleReplicas = 1024;
+
+__device__ __forceinline__ uint32_t entry_tag(uint64_t nonce, int i) {
+  return static_cast<uint32_t>((i & 1) != 0 ? nonce >> 32 : nonce);
+}
+
+// A value that every lane of the wavefront holds alike, as the compiler can
+// know it.
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(x));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(x >> 32));
+  return uint64_t(hi) << 32 | lo;
+}
+
+// Replica r's constants from its entry, if the scalar cache has them.
+template <int N, typename T>
+__device__ __forceinline__ bool entry_cached(const Single<T>& one, uint32_t r,
+                                             double (&out)[N]) {
+  const auto* e = reinterpret_cast<const __attribute__((address_space(4))) uint64_t*>(
+      reinterpret_cast<uintptr_t>(one.entries + kEntryWords * r));
+  uint64_t word[2 * N];
+#pragma unroll
+  for (int i = 0; i < 2 * N; ++i) word[i] = e[i];
+  uint32_t other = 0;
+#pragma unroll
+  for (int i = 0; i < 2 * N; ++i) {
+    other |= static_cast<uint32_t>(word[i] >> 32) ^ entry_tag(one.nonce, i);
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    out[k] = __builtin_bit_cast(double, word[2 * k] << 32 | (word[2 * k + 1] & 0xFFFFFFFFu));
+  }
+  return other == 0;
+}
+
+// The same from memory, one access for the wavefront: lane i reads word
+// i % 2N (entry_load), and what it read is looked at later (entry_is).
+template <int N, typename T>
+__device__ __forceinline__ uint64_t entry_load(const Single<T>& one, uint32_t r) {
+  return __hip_atomic_load(one.entries + kEntryWords * r + __lane_id() % (2 * N),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int N, typename T>
+__device__ __forceinline__ bool entry_is(const Single<T>& one, uint64_t word, double (&out)[N]) {
+  const int i = static_cast<int>(__lane_id()) % (2 * N);
+  const bool mine = static_cast<uint32_t>(word >> 32) == entry_tag(one.nonce, i);
+  if (__ballot(mine) != ~uint64_t(0)) return false;
+  const uint32_t half = static_cast<uint32_t>(word);
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const uint64_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(half, 2 * k));
+    const uint32_t lo = __builtin_amdgcn_readlane(half, 2 * k + 1);
+    out[k] = __builtin_bit_cast(double, hi << 32 | lo);
+  }
+  return true;
+}
+
+// Every vector memory operation the wavefront has issued is done before any
+// later one starts. An agent-scope store is done when the memory that all XCDs
+// share has it, so between two of them this orders what other workgroups can
+// see. A release fence would also write the XCD's L2 back (and an acquire
+// invalidate it), for data that went through it; none did here, and with those
+// in every workgroup's path the 8 x 265,484 Adam call took 40 us.
+__device__ __forceinline__ void memory_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+template <typename T>
+using StepBits = std::conditional_t<sizeof(T) == 2, uint16_t,
+                                    std::conditional_t<sizeof(T) == 4, uint32_t, uint64_t>>;
+
+// x advanced by a call on an active replica, as bump_steps_kernel stores it.
+template <typename T>
+__device__ __forceinline__ T bumped(T x, bool bump) {
+  return bump ? narrow<T>(widen(x) + op_t<T>(1)) : x;
+}
+
+// Replica r's step as the scalar cache has it, from before the bump or from
+// after it. It is read once: step_is, before the look into the entry, waits for
+// it and keeps the compiler from reading it again after.
+template <typename T>
+__device__ __forceinline__ StepBits<T> step_read(const T* steps, uint32_t r) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(steps + r);
+  if constexpr (sizeof(T) == 2) {
+    const auto* word =
+        reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(at & ~uintptr_t(3));
+    return static_cast<uint16_t>(*word >> (8 * (at & 2)));
+  } else {
+    return *reinterpret_cast<const __attribute__((address_space(4))) StepBits<T>*>(at);
+  }
+}
+template <typename B>
+__device__ __forceinline__ B step_is(B x) {
+  if constexpr (sizeof(B) == 8) {
+    asm volatile("" : "+s"(x)::"memory");
+    return x;
+  } else {
+    uint32_t w = x;
+    asm volatile("" : "+s"(w)::"memory");
+    return static_cast<B>(w);
+  }
+}
+
+// The constants of a replica every lane of the wavefront works on, in a
+// single-launch call. `x`: the step as read (step_read). `head`: this wavefront
+// is the replica's head and makes them known.
+template <typename P>
+__device__ __forceinline__ void single_constants(const Vectors<typename P::T>& v, uint32_t r,
+                                                 StepBits<typename P::T> x, bool head,
+                                                 double (&w)[P::kConstants]) {
+  using T = typename P::T;
+  using Bits = StepBits<T>;
+  constexpr int N = P::kConstants;
+  const Single<T>& one = v.one;
+  const T read = __builtin_bit_cast(T, step_is(x));
+  const bool look = !head && P::needs_entry(read, one.bump);
+  const bool late = look && blockIdx.x >= one.early;
+  if (late && entry_cached(one, r, w)) return;
+  const uint64_t word = look ? entry_load<N>(one, r) : 0;
+  if (late && entry_is(one, word, w)) return;
+  const T step = bumped(read, one.bump);
+  typename P::Rep rep;
+  uniform_derive<P>(v, r, static_cast<double>(widen(step)), rep);
+  P::constants(rep, w);
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    w[k] = __builtin_bit_cast(double, uniform64(__builtin_bit_cast(uint64_t, w[k])));
+  }
+  if (look) entry_is(one, word, w);
+  if (head && threadIdx.x == 0) {
+    uint64_t* const e = one.entries + kEntryWords * r;
+#pragma unroll
+    for (int i = 0; i < 2 * N; ++i) {
+      const uint64_t half = __builtin_bit_cast(uint64_t, w[i / 2]) >> (i % 2 == 0 ? 32 : 0);
+      const uint64_t word = uint64_t(entry_tag(one.nonce, i)) << 32 | (half & 0xFFFFFFFFu);
+      __hip_atomic_store(e + i, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (one.bump) {
+      memory_done();
+      __hip_atomic_store(reinterpret_cast<Bits*>(one.steps + r), __builtin_bit_cast(Bits, step),
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+// The same in a call with its preparation (or bump) in a launch before.
+template <typename P, bool PRE>
+__device__ __forceinline__ void call_constants(const Vectors<typename P::T>& v, uint32_t r,
+                                               double (&w)[P::kConstants]) {
+  if constexpr (PRE) {
+#pragma unroll
+    for (int k = 0; k < P::kConstants; ++k) w[k] = v.pre[kPreStride * r + k];
+  } else {
+    typename P::Rep rep;
+    P::derive(v, r, step_at(v.steps, r), rep);
+    P::constants(rep, w);
+  }
+}
+
+// What a head does besides: the zero result, and a frozen replica's step (the
+// bump adds zero to it, as bump_steps_kernel does).
+template <typename T>
+__device__ __forceinline__ void single_head(const Single<T>& one, uint32_t r, bool active) {
+  if (threadIdx.x != 0) return;
+  if (r == 0 && one.out_zero != nullptr) *one.out_zero = narrow<T>(op_t<T>(0));
+  if (!active && one.bump) one.steps[r] = narrow<T>(widen(one.steps[r]) + op_t<T>(0));
 }
 
 // Elements per streaming tile: the workgroup's threads x the policy's packs
@@ -1335,11 +1616,14 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
   uint32_t r;
   int64_t t0;
   stream_tile_of_block<kStreamTile>(a.g, r, t0);
-  if constexpr (stream_scalar_mask<P, SMALL>()) {
-    if (!mask_byte_scalar(a.vec.mask, r)) return;
-  } else {
-    if (!a.vec.mask[r]) return;
-  }
+  const bool active = stream_scalar_mask<P, SMALL>() ? mask_byte_scalar(a.vec.mask, r)
+                                                     : a.vec.mask[r] != 0;
+  // In a single-launch call the row's tile 0 is its replica's head.
+  constexpr bool kSingle = PRE || P::kPreWords == 0;
+  const bool single = kSingle && a.vec.one.nonce != 0;
+  const bool is_head = single && t0 == 0 && threadIdx.x < 64;
+  if (is_head) single_head(a.vec.one, r, active);
+  if (!active) return;
 
   // A row's tiles k >= 1 start at its first kStreamTile-element boundary, so
   // no tile straddles one (on rows whose length is not a multiple of the tile,
@@ -1356,7 +1640,10 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
   // the single elements [0, pre) and [body_end, width).
   const auto run = [&](auto head_tile, int64_t first, int64_t packs_left, int64_t pre,
                        int64_t body_end) __attribute__((always_inline)) {
-    const bool load_state = P::reads_state(a.vec, r);
+    const StepBits<T> x = single ? step_read(a.vec.one.steps, r) : StepBits<T>(0);
+    const bool load_state = single
+                                ? P::may_read_state(__builtin_bit_cast(T, x), a.vec.one.bump)
+                                : P::reads_state(a.vec, r);
     T* const pbase = pg_row<P>(a.x, 0, r);
     const T* const gbase = pg_row<P>(a.x, 1, r);
     S* sbase[SS];
@@ -1395,7 +1682,18 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
       }
     }
     typename P::Rep rep;
-    uniform_prologue<P, PRE>(a.vec, r, rep);
+    if constexpr (kSingle) {
+      P::hypers(a.vec, r, rep);
+      double w[P::kConstants];
+      if (single) {
+        single_constants<P>(a.vec, r, x, is_head, w);
+      } else {
+        call_constants<P, PRE>(a.vec, r, w);
+      }
+      P::set(w, rep);
+    } else {
+      uniform_prologue<P, PRE>(a.vec, r, rep);
+    }
     const auto store_packs = [&](int u, int64_t i) {
       store_stream<NT>(prow + i, vp[u]);
 #pragma unroll
@@ -1471,7 +1769,7 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
   const int64_t head_packs = (head - pre) / KP;
   const int64_t body_end =
       head < width ? head + (width - head) / KP * KP : pre + head_packs * KP;
-  if (head_packs > 0 || pre > 0 || body_end < width) {
+  if (head_packs > 0 || pre > 0 || body_end < width || is_head) {
     run(std::true_type{}, pre, head_packs, pre, body_end);
   }
 }
@@ -1704,7 +2002,7 @@ __global__ __launch_bounds__(kColThreads) void column_kernel(ColArgs<P> a) {
     return;
   }
   typename P::Rep rep;
-  P::template prologue<PRE>(a.vec, static_cast<uint32_t>(r), rep);
+  prologue<P, PRE>(a.vec, static_cast<uint32_t>(r), rep);
   const bool load_state = P::reads_state(a.vec, static_cast<uint32_t>(r));
   const int64_t t_first = int64_t(cblk) * a.g.cpi * kColIters + cc;
   if (nt) {
@@ -1811,8 +2109,25 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
   // config 5's per-parameter gradients).
   constexpr int KP = stream_pack<T, S>();
   const uint32_t tiles_per_row = a.seg.tile0[a.seg.n];
-  const uint32_t r = blockIdx.x / tiles_per_row;
-  const uint32_t local = blockIdx.x - r * tiles_per_row;
+  // A single-launch call's first workgroups are the replicas' heads, which only
+  // make the constants known.
+  constexpr bool kSingle = PRE || P::kPreWords == 0;
+  const bool single = kSingle && a.k.vec.one.nonce != 0;
+  if (blockIdx.x < a.k.g.heads) {
+    const uint32_t r = blockIdx.x;
+    const bool active = mask_byte_scalar(a.k.vec.mask, r);
+    if (threadIdx.x < 64) {
+      single_head(a.k.vec.one, r, active);
+      if (active) {
+        double w[P::kConstants];
+        single_constants<P>(a.k.vec, r, step_read(a.k.vec.one.steps, r), true, w);
+      }
+    }
+    return;
+  }
+  const uint32_t block = blockIdx.x - a.k.g.heads;
+  const uint32_t r = block / tiles_per_row;
+  const uint32_t local = block - r * tiles_per_row;
   const bool write_grad = a.k.x.data[1] != nullptr;
   const bool active = segment_scalar_mask_of<P>::value ? mask_byte_scalar(a.k.vec.mask, r)
                                                         : a.k.vec.mask[r] != 0;
@@ -1864,8 +2179,24 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
   }
 
   typename P::Rep rep;
-  P::template prologue<PRE>(a.k.vec, r, rep);
-  const bool load_state = P::reads_state(a.k.vec, r);
+  const StepBits<T> x = single ? step_read(a.k.vec.one.steps, r) : StepBits<T>(0);
+  const bool load_state = single
+                              ? P::may_read_state(__builtin_bit_cast(T, x), a.k.vec.one.bump)
+                              : P::reads_state(a.k.vec, r);
+  const auto constants = [&]() __attribute__((always_inline)) {
+    if constexpr (kSingle) {
+      P::hypers(a.k.vec, r, rep);
+      double w[P::kConstants];
+      if (single) {
+        single_constants<P>(a.k.vec, r, x, false, w);
+      } else {
+        call_constants<P, PRE>(a.k.vec, r, w);
+      }
+      P::set(w, rep);
+    } else {
+      prologue<P, PRE>(a.k.vec, r, rep);
+    }
+  };
   const T zero = narrow<T>(op_t<T>(0));
 
   T* const prow = pg_row<P>(a.k.x, 0, r) + col * a.k.x.stride_t[0];
@@ -1894,6 +2225,7 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
   };
 
   if (!vec) {
+    constants();
     const int64_t cnt = imin(kSegTile, numel - j0);
     for (int64_t j = j0 + threadIdx.x; j < j0 + cnt; j += NTH) one(j);
     return;
@@ -1930,6 +2262,7 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
       }
     }
   }
+  constants();
   with_variant<P>(rep, [&](const typename P::Rep& rp) {
     with_maximize<P>(a.k.maximize, [&](bool mx) {
 #pragma unroll
@@ -2057,7 +2390,9 @@ __global__ __launch_bounds__(kThreads) void prep_kernel(Vectors<typename P::T> v
       steps[r] = narrow<T>(widen(steps[r]) + one);
     }
     if (active) {
-      P::precompute(v, static_cast<uint32_t>(r), pre + kPreStride * r);
+      typename P::Rep rep;
+      P::derive(v, static_cast<uint32_t>(r), step_at(v.steps, static_cast<uint32_t>(r)), rep);
+      P::constants(rep, pre + kPreStride * r);
     }
   }
   if (out_zero != nullptr && r == 0) {
@@ -2303,18 +2638,22 @@ bool walk_fits(SegmentWalk w, int64_t R, int64_t tile, bool vec_rows, Segments<T
   return true;
 }
 
-// Launches `kernel` once per chunk of the walk.
+// Launches `kernel` once per chunk of the walk; the first launch with `*heads`
+// more workgroups in front (a field of `a`).
 template <typename T, typename Args, typename Kernel>
 int launch_walk(SegmentWalk w, int64_t R, int64_t tile, bool vec_rows, Args& a, Segments<T>& seg,
-                Kernel kernel, hipStream_t stream, uint32_t lds = 0, int threads = kThreads) {
+                Kernel kernel, hipStream_t stream, uint32_t lds = 0, int threads = kThreads,
+                uint32_t* heads = nullptr) {
   int64_t blocks;
   while ((blocks = next_chunk<T>(w, R, tile, vec_rows, seg, threads)) != 0 || seg.n > 0) {
     if (blocks < 0) return kInvalid;
     if (blocks == 0) continue;
+    if (heads != nullptr) blocks += *heads;
     hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(blocks)), dim3(threads), lds, stream,
                        a);
     const int err = static_cast<int>(hipGetLastError());
     if (err != 0) return err;
+    if (heads != nullptr) *heads = 0;  // in the call's first launch only
   }
   return 0;
 }
@@ -2372,8 +2711,49 @@ bool fill_kargs(const Call& c, int nbufs, KArgs<P>& a, bool grad_optional) {
   a.vec.mask = c.mask;
   a.vec.pre = uses_workspace<P>(c) ? static_cast<const double*>(c.ws) : nullptr;
   a.vec.ilp_rows = ilp_rows_rule<P>(a.x, c.T);
+  a.vec.one = Single<T>{0, nullptr, nullptr, nullptr, 0, false};
   a.maximize = (c.flags & TS_MAXIMIZE) != 0;
   return true;
+}
+
+// A launch's identity for the entries of its workspace: both 32-bit halves
+// step through all their values, so neither repeats within 2^32 launches; the
+// start differs from process to process.
+inline uint64_t next_nonce() {
+  static std::atomic<uint64_t> count{
+      static_cast<uint64_t>(std::chrono::steady_clock::now().time_since_epoch().count())};
+  uint64_t nonce;
+  do {
+    const uint64_t c = count.fetch_add(1, std::memory_order_relaxed);
+    const uint32_t lo = static_cast<uint32_t>(c) * 0x9E3779B1u;
+    const uint32_t hi =
+        static_cast<uint32_t>(c) * 0x85EBCA77u + static_cast<uint32_t>(c >> 32) * 0xC2B2AE3Du;
+    nonce = uint64_t(hi) << 32 | lo;
+  } while (nonce == 0);
+  return nonce;
+}
+
+inline bool stream_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
+// Whether a call with streamable operands runs as one launch: a workspace that
+// holds the entries, few enough replicas, and no capture.
+inline bool single_launch(const Call& c) {
+  return c.ws != nullptr && c.R <= kSingleReplicas &&
+         c.ws_bytes / (kEntryWords * sizeof(uint64_t)) >= static_cast<uint64_t>(c.R) &&
+         !stream_capturing(c.stream);
+}
+
+template <typename T>
+Single<T> single_of(const Call& c, uint32_t early) {
+  return Single<T>{next_nonce(), static_cast<uint64_t*>(c.ws), static_cast<T*>(c.steps),
+                   static_cast<T*>(c.out_zero), early, (c.flags & TS_BUMP_STEPS) != 0};
 }
 
 template <typename P>
@@ -2390,7 +2770,8 @@ int launch_prep(const Call& c, const Vectors<typename P::T>& vec) {
   return static_cast<int>(hipGetLastError());
 }
 
-// Validation, then the preparation launch (the optional bump and the zero
+// Validation, then (unless `prepare` made it a single launch, vec.one) the
+// preparation launch (the optional bump and the zero
 // result; with a workspace also the per-replica constants), then `launch`
 // when there is any work. Every check happens before the first enqueue, so an
 // invalid call changes nothing. Empty tensors may carry null data pointers, so
@@ -2399,7 +2780,7 @@ int launch_prep(const Call& c, const Vectors<typename P::T>& vec) {
 // in `vec`) when there is at least one element. A workspace must hold
 // kPreStride doubles per replica and be 8-byte aligned.
 template <typename P, typename Prepare, typename Launch>
-int run_step(const Call& c, const Vectors<typename P::T>& vec, Prepare&& prepare,
+int run_step(const Call& c, Vectors<typename P::T>& vec, Prepare&& prepare,
              Launch&& launch) {
   using T = typename P::T;
   if (c.bufs == nullptr || c.R < 0 || c.T < 0 ||
@@ -2415,7 +2796,9 @@ int run_step(const Call& c, const Vectors<typename P::T>& vec, Prepare&& prepare
   if (work && !prepare()) {
     return kInvalid;
   }
-  if (work && uses_workspace<P>(c)) {
+  if (work && vec.one.nonce != 0) {
+    // One launch: the update's heads do what the preparation would.
+  } else if (work && uses_workspace<P>(c)) {
     const int err = launch_prep<P>(c, vec);
     if (err != 0) return err;
   } else if ((c.flags & TS_BUMP_STEPS) != 0 && c.R > 0) {
@@ -2491,6 +2874,9 @@ int launch_dense(const Call& c, int nbufs) {
     if (!make_grid(c.R, c.T, tile, a.g, blocks, threads, streamable)) return false;
     a.g.res0 = res0;
     a.g.rmod = rmod;
+    if (streamable && single_launch(c)) {
+      a.vec.one = single_of<typename P::T>(c, kEarlyBlocks);
+    }
     return true;
   };
   return run_step<P>(c, a.vec, prepare, [&]() -> int {
@@ -2561,9 +2947,16 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
     a.k.g = Grid{c.T, 0, 0, 0, 0, 0, 0, 0};
     vec_rows = rows_streamable<P>(a.k.x, nbufs, a.k.g.res0, a.k.g.rmod);
     const int nth = pre ? segment_threads<P, true>() : segment_threads<P, false>();
-    return walk_fits<T>(walk, c.R, tile, vec_rows, a.seg, nth);
+    if (!walk_fits<T>(walk, c.R, tile, vec_rows, a.seg, nth)) return false;
+    // No more workgroups than this, heads included: T / tile, the last tile of
+    // every segment and of every gap, and one head, per replica.
+    const uint64_t most = static_cast<uint64_t>(c.R) * (c.T / tile + 2 * n_segs + 3);
+    if (grid_fits(most, nth) && single_launch(c)) a.k.vec.one = single_of<T>(c, 0);
+    return true;
   };
   return run_step<P>(c, a.k.vec, prepare, [&]() -> int {
+    if (a.k.vec.one.nonce != 0) a.k.g.heads = static_cast<uint32_t>(c.R);
+    uint32_t* const heads = &a.k.g.heads;
     const bool same_phase =
         rows_same_phase<P>(a.k.x, nbufs, stream_pack<typename P::T, typename P::S>());
     if constexpr (P::kPreWords > 0) {
@@ -2574,16 +2967,16 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
         const uint32_t lds =
             c.R * c.T >= kCapMinElems ? segment_lds_pre_of<P>::value : 0u;
         return same_phase ? launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg,
-                                           segment_kernel<P, false, true>, c.stream, lds, nth)
+                                           segment_kernel<P, false, true>, c.stream, lds, nth, heads)
                           : launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg,
-                                           segment_kernel<P, true, true>, c.stream, lds, nth);
+                                           segment_kernel<P, true, true>, c.stream, lds, nth, heads);
       }
     }
     constexpr int nth = segment_threads<P, false>();
     return same_phase ? launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg,
-                                       segment_kernel<P, false, false>, c.stream, 0, nth)
+                                       segment_kernel<P, false, false>, c.stream, 0, nth, heads)
                       : launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg,
-                                       segment_kernel<P, true, false>, c.stream, 0, nth);
+                                       segment_kernel<P, true, false>, c.stream, 0, nth, heads);
   });
 }
 

@@ -11,6 +11,7 @@
 #include <algorithm>
 
 #include "optim_dispatch.h"
+#include "optim_internal.h"
 
 namespace churten {
 namespace {
@@ -52,6 +53,12 @@ int ts_version(void) { return 200; }
 
 size_t ts_workspace_bytes(int64_t R) {
   return R > 0 ? static_cast<size_t>(R) * churten::kPreStride * sizeof(double) : 0;
+}
+
+size_t ts_single_launch_bytes(int64_t R) {
+  return R > 0 && R <= churten::kSingleReplicas
+             ? static_cast<size_t>(R) * churten::kEntryWords * sizeof(uint64_t)
+             : 0;
 }
 
 int ts_bump_steps(ts_dtype dtype, void* state_steps, const uint8_t* active_mask,

@@ -30,9 +30,11 @@
 // params (all of them, TS_STATE_BF16); the reference rejects mixed dtypes.
 //
 // The common case (steps in the param dtype, a bool mask, contiguous (R,)
-// vectors) costs two launches: the preparation (step bump, zero result and,
-// for Adam and Adagrad, the per-replica constants into a workspace) and the
-// update. Anything else is first normalised with ATen ops.
+// vectors, unit inner strides) costs one launch: the update, which bumps the
+// steps, clears the result and passes the per-replica constants through a
+// workspace on the way. Other strides, many replicas and graph capture take two
+// (a preparation or bump, then the update). Anything else is first normalised
+// with ATen ops.
 
 #include <Python.h>
 
@@ -49,6 +51,7 @@
 #include <vector>
 
 #include "../../include/churten_optim.h"
+#include "optim_internal.h"
 
 namespace churten {
 namespace {
@@ -142,9 +145,10 @@ hipStream_t current_stream(const at::Tensor& params) {
 // Everything a launcher needs besides the (R, T) operand table: the step
 // counter (bumped by the launcher when TS_BUMP_STEPS is set), the mask, the
 // normalised hyperparameter vectors, the fresh zero result and, when there is
-// work, the workspace for the per-replica constants (ts_workspace_bytes(R)
-// bytes from torch's caching allocator on the current stream: no device
-// allocation once the allocator is warm, and stream-ordered reuse).
+// work, the workspace (room for a single launch where R allows one, else for
+// the per-replica constants of a policy that has any; from torch's caching
+// allocator on the current stream: no device allocation once the allocator is
+// warm, and stream-ordered reuse).
 struct Prepared {
   ts_dtype dtype;
   uint32_t flags;
@@ -166,7 +170,7 @@ struct Prepared {
 Prepared prepare(const at::Tensor& params, at::Tensor& state_steps,
                  const at::Tensor& active_mask, std::initializer_list<const at::Tensor*> hyp,
                  std::initializer_list<const char*> names, uint32_t flags, const char* op,
-                 bool want_ws = true) {
+                 bool has_constants = true) {
   check_vec(params, state_steps, op, "state_steps");
   check_vec(params, active_mask, op, "active_mask");
   auto name = names.begin();
@@ -191,9 +195,10 @@ Prepared prepare(const at::Tensor& params, at::Tensor& state_steps,
   p.out = at::empty({}, params.options());
   p.R = params.size(0);
   p.T = params.size(1);
-  if (want_ws && p.R > 0 && p.T > 0) {
-    p.ws = at::empty({static_cast<int64_t>(ts_workspace_bytes(p.R))},
-                     params.options().dtype(at::kByte));
+  size_t bytes = p.T > 0 ? ts_single_launch_bytes(p.R) : 0;
+  if (bytes == 0 && has_constants && p.T > 0) bytes = ts_workspace_bytes(p.R);
+  if (bytes > 0) {
+    p.ws = at::empty({static_cast<int64_t>(bytes)}, params.options().dtype(at::kByte));
   }
   p.stream = current_stream(params);
   return p;
@@ -301,12 +306,17 @@ at::Tensor sgd_step_gpu(at::Tensor params, at::Tensor grads,
                              {"lr", "momentum", "dampening", "weight_decay"},
                              sflag | (nesterov ? TS_NESTEROV : 0u) |
                                  (maximize ? TS_MAXIMIZE : 0u),
-                             op, /*want_ws=*/false);
+                             op, /*has_constants=*/false);
   const ts_rt_buf bufs[3] = {rt_buf(params), rt_buf(grads),
                              momentum_buffers.has_value() ? rt_buf(*momentum_buffers) : kNoBuf};
-  check_status(ts_sgd_step(bufs, p.dtype, p.steps.data_ptr(), p.h(0), p.h(1), p.h(2), p.h(3),
-                           p.m(), p.R, p.T, p.flags, p.out.data_ptr(), p.stream),
-               op);
+  check_status(
+      p.has_ws()
+          ? ts_sgd_step_ws(bufs, p.dtype, p.steps.data_ptr(), p.h(0), p.h(1), p.h(2), p.h(3),
+                           p.m(), p.R, p.T, p.flags, p.out.data_ptr(), p.ws_ptr(), p.ws_bytes(),
+                           p.stream)
+          : ts_sgd_step(bufs, p.dtype, p.steps.data_ptr(), p.h(0), p.h(1), p.h(2), p.h(3), p.m(),
+                        p.R, p.T, p.flags, p.out.data_ptr(), p.stream),
+      op);
   return p.out;
 }
 
@@ -434,13 +444,19 @@ at::Tensor sgd_step_segments_gpu(at::Tensor params, at::TensorList grads, at::In
                              {"lr", "momentum", "dampening", "weight_decay"},
                              sflag | (nesterov ? TS_NESTEROV : 0u) |
                                  (maximize ? TS_MAXIMIZE : 0u),
-                             op, /*want_ws=*/false);
+                             op, /*has_constants=*/false);
   const ts_rt_buf bufs[3] = {rt_buf(params), grads_out.has_value() ? rt_buf(*grads_out) : kNoBuf,
                              momentum_buffers.has_value() ? rt_buf(*momentum_buffers) : kNoBuf};
-  check_status(ts_sgd_step_segments(bufs, st.segs.data(), static_cast<int>(st.segs.size()),
-                                    p.dtype, p.steps.data_ptr(), p.h(0), p.h(1), p.h(2), p.h(3),
-                                    p.m(), p.R, p.T, p.flags, p.out.data_ptr(), p.stream),
-               op);
+  const int n = static_cast<int>(st.segs.size());
+  check_status(
+      p.has_ws()
+          ? ts_sgd_step_segments_ws(bufs, st.segs.data(), n, p.dtype, p.steps.data_ptr(),
+                                    p.h(0), p.h(1), p.h(2), p.h(3), p.m(), p.R, p.T, p.flags,
+                                    p.out.data_ptr(), p.ws_ptr(), p.ws_bytes(), p.stream)
+          : ts_sgd_step_segments(bufs, st.segs.data(), n, p.dtype, p.steps.data_ptr(), p.h(0),
+                                 p.h(1), p.h(2), p.h(3), p.m(), p.R, p.T, p.flags,
+                                 p.out.data_ptr(), p.stream),
+      op);
   return p.out;
 }
 

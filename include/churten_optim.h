@@ -180,13 +180,17 @@ int ts_adagrad_step_segments(const ts_rt_buf* bufs, const ts_segment* grads, int
  * shorter tile per workgroup: the config-5 Adam step (128 x 25.2M float32)
  * 6.46-6.51 TB/s against 6.14-6.18 for ts_adam_step on the same buffers.
  *   workspace:       device memory of at least ts_workspace_bytes(R) bytes,
- *                    8-byte aligned, not NULL. It is scratch: nothing is read
- *                    from it before the call writes it, and its contents after
- *                    the call mean nothing. It must not be shared with another
+ *                    8-byte aligned, not NULL. It is scratch: its contents
+ *                    before and after the call mean nothing. It must not be shared with another
  *                    call that may run at the same time (another stream).
  *   workspace_bytes: its size; smaller than ts_workspace_bytes(R) is an
  *                    invalid argument.
- * Still two launches per call (preparation, update), as without a workspace.
+ * Two launches per call (preparation, update), as without a workspace. With a
+ * workspace of 128 R bytes or more, R <= 1024, unit inner strides and no
+ * capture under way on the stream, the call is one launch: the update bumps the
+ * steps and passes the constants on itself, with the same results (the
+ * preparation launch costs 2-3.5 us of GPU time). It then also reads what the
+ * workspace held before, to tell that it is not its own.
  * These replace the same reference interfaces as ts_adam_step, ts_adagrad_step
  * and their segmented forms (stubs.cpp:25-41, 61-72; cuda/adam.cu:99-122 and
  * cuda/adagrad.cu:141-148 are the per-block prologues whose constants the
