@@ -35,7 +35,7 @@ int scatter(const ts_segment* segs, int n_segs, void* dst, int64_t dst_stride_r,
     return s.numel > 0;
   });
   if ((any && dst == nullptr) ||
-      !walk_fits<T>(walk, R, scatter_tile<T>(), vec_rows, a.seg, kScatterThreads)) {
+      !walk_fits(walk, R, scatter_tile<T>(), kScatterThreads)) {
     return kInvalid;
   }
   return launch_walk<T>(walk, R, scatter_tile<T>(), vec_rows, a, a.seg, scatter_kernel<T>, stream,

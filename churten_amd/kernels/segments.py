@@ -6,7 +6,7 @@ the fused update (src/torchstrap/optimizer/grad_transform.py:29-30). These ops
 (C++/HIP, churten_amd/csrc) take the per-parameter gradients directly:
 
 * ``scatter_grads_(dst, grads, cols)`` -- the whole scatter in one launch per
-  64 parameters;
+  64 parameters or more;
 * ``{adam,sgd,adagrad}_step_segments_(params, grads, cols, grads_out, ...)``
   -- the update reads each parameter's gradient where it lies; ``grads_out``
   (optional) receives the consolidated gradient on the way through. Every

@@ -152,8 +152,8 @@ int ts_adagrad_step(const ts_rt_buf* bufs, ts_dtype dtype, void* state_steps,
  * segment covers take their gradient from it; with NULL they take zero. Element
  * math and flags as the consolidated forms, so every column ends up identical
  * to ts_scatter_segments into bufs[1] (or into a zeroed buffer) followed by
- * ts_*_step. One launch per 64 table entries (segments and the gaps between
- * them), plus the bump. */
+ * ts_*_step. One launch per 128 table entries (segments and the gaps
+ * between them), plus the bump. */
 int ts_adam_step_segments(const ts_rt_buf* bufs, const ts_segment* grads, int n_grads,
                           ts_dtype dtype, void* state_steps, const void* lr,
                           const void* beta1, const void* beta2, const void* eps,
@@ -236,7 +236,7 @@ int ts_adam_step_noalloc(const ts_rt_buf* bufs, ts_dtype dtype, void* state_step
                          const void* weight_decay, const uint8_t* active_mask, int64_t R,
                          int64_t T, uint32_t flags, void* out_zero, void* stream);
 
-/* Gradient scatter in one launch per 64 segments: copies every segment, all R
+/* Gradient scatter in one launch per 64 segments or more: copies every segment, all R
  * rows, into its columns of the (R, cols) buffer dst (row stride dst_stride_r,
  * unit column stride); other columns are not written. Replaces the
  * per-parameter copies of grad_transform.py:29. */
