@@ -431,14 +431,30 @@ constexpr bool kHalfAll = std::is_same<T, _Float16>::value && std::is_same<S, _F
 constexpr int64_t kCapMinElems = int64_t(8192) * 512;
 
 // Launches whose (R, T) operands take at most this many bytes run the SMALL
-// streaming shape (plain accesses, the policy's kStreamUnrollSmall, no cap):
-// the MI355X's 256 MB MALL then keeps them between back-to-back steps.
-// Measured on configs 1-4 (prep + update through the C ABI, 200 launches, 5
-// rounds): config 1 (34 MB of Adam operands) 11.7 us plain with 2 packs
-// against 13.0 non-temporal; config 3 (209 MB, SGD) 32.0 us plain with 1 pack
-// (2 / 4 / 8 packs: 33.9 / 32.6 / 32.2) against 35.8; configs 2 and 4 (531 /
-// 419 MB) lose 11-16% with plain accesses, so they stay non-temporal.
-constexpr int64_t kMallBytes = int64_t(256) << 20;
+// streaming shape (plain accesses, the policy's kStreamUnrollSmall, no cap): the
+// MI355X's 256 MB MALL then keeps them from one step to the next, with room for
+// what a training step touches in between. Whole calls on three states in turn
+// (so three times the operands pass between two steps of one), plain against
+// non-temporal, same process: float32 Adam at 34 / 51 / 85 / 102 / 119 / 136 /
+// 238 MB 11.9 / 16.1 / 25.3 / 31.1 / 39.9 / 47.9 / 80.3 us against 12.9 / 17.4 /
+// 26.5 / 30.4 / 34.7 / 39.2 / 65.9, and every other optimizer and type crosses
+// between 84 and 131 MB too (16-bit Adagrad at 130-200). With one state alone,
+// plain accesses win up to 209 MB (config 3 32.0 us against 35.8), but then
+// nothing else may pass through the cache between steps.
+constexpr int64_t kMallBytes = int64_t(100) << 20;
+
+// The smallest launches of some policies take the large shape too
+// (kStreamSmallFrom, bytes of operands): its shorter tiles spread the launch
+// over more wavefronts. Same A/B, large shape against SMALL: Adam at 10-26 MB
+// float32 +10-14% (34 MB: -8%), with bfloat16 moments +3-8%, float16 +10-18%,
+// bfloat16 +21% (35 MB +9%, 70 MB 0), float64 +11-16%; 16-bit SGD +10-21% to 39
+// MB (58 MB: -3%); float64 SGD and Adagrad and float32 Adagrad +3-15% at 6-13
+// MB, -5% to +3% at 26. Float32 SGD (-3% to 0) and 16-bit Adagrad (-15% to -34%)
+// keep SMALL.
+template <typename T>
+constexpr int64_t small_from(int64_t wide, int64_t narrow) {
+  return (sizeof(T) == 2 ? narrow : wide) << 20;
+}
 
 // Launches above the MALL with at most kMidBytes of (R, T) operands reserve
 // each policy's kStreamLdsMid instead of its large-launch cap (with a
@@ -646,7 +662,8 @@ struct AdamPolicy {
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(2, 1, 1, 2);
   static constexpr bool kScalarMaskSmall =
       !kFp32State<T, S> && !std::is_same<T, double>::value;
-  static constexpr int64_t kStreamSmallBytes = kMallBytes;
+  static constexpr int64_t kStreamSmallFrom =
+      std::is_same<T, bf16_t>::value ? int64_t(48) << 20 : int64_t(28) << 20;
   static constexpr int kStreamPack = stream_pack<T, S>();
   static constexpr int kSegmentUnroll = stream_unroll<T, S>(2, 4, 4, 2);
   static constexpr int kSegmentThreads = kThreads;
@@ -781,7 +798,8 @@ struct SgdPolicy {
   // and 6.88-6.93 for 256; with the scalar read 256 threads ran 2.2% ahead of
   // 128 (same-process A/B, 10 rounds).
   static constexpr int kStreamBlockSmall = kFp32State<T, S> ? 256 : kStreamThreads;
-  static constexpr int64_t kStreamSmallBytes = kMallBytes;
+  static constexpr int64_t kStreamSmallFrom =
+      small_from<T>(std::is_same<T, double>::value ? 16 : 0, 48);
   static constexpr int kStreamPack = stream_pack<T, S>();
   // Segmented float32 updates: one-wavefront workgroups, one pack, the flag
   // read through the scalar cache (same-process A/B on config 5's twelve
@@ -863,7 +881,7 @@ struct AdagradPolicy {
   // +9%; two packs +5%).
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(2, 1, 1, 2);
   static constexpr bool kScalarMaskSmall = sizeof(T) == 2;
-  static constexpr int64_t kStreamSmallBytes = kMallBytes;
+  static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
   static constexpr int kStreamPack = stream_pack<T, S>();
   // Segmented float32 updates with a workspace: one-wavefront workgroups, one
   // pack, the scalar flag read, uncapped (same-process A/B on config 5's
@@ -987,7 +1005,7 @@ struct AdagradF32Policy {
   static constexpr int kStreamUnrollPre = stream_unroll<T, S>(1, 1, 1, 2);
   static constexpr bool kScalarMask = std::is_same<T, float>::value;
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(2, 1, 4, 2);
-  static constexpr int64_t kStreamSmallBytes = kMallBytes;
+  static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
   static constexpr int kStreamPack = stream_pack<T, S>();
   // Segmented with a workspace: one-wavefront workgroups, one pack, the
   // scalar flag read, as Adagrad (config 5's per-parameter gradients,
@@ -2047,7 +2065,7 @@ struct SegArgs {
                // k.g.res0 / rmod: the params rows' phase
   Segments<typename P::T> seg;
 };
-static_assert(sizeof(KArgs<AdamPolicy<double, true, true>>) + sizeof(Segments<double>) <= 4096,
+static_assert(sizeof(SegArgs<AdamPolicy<double, true, true>>) <= 4096,
               "a launch's arguments");
 
 __device__ __forceinline__ int segment_of_tile(const uint32_t* tile0, int n, uint32_t t) {
@@ -2102,9 +2120,27 @@ __device__ __forceinline__ void seg_singles(const SegTile& t, int64_t numel, Fn&
   }
 }
 
+// Plain accesses in a segmented launch, where the MALL gains by them (CACHE);
+// the rest is non-temporal. Whole calls on three states in turn, same-process
+// A/B:
+//   2: every load, for launches whose operands take kSegCacheMin to kMallBytes
+//   (stores of parameters and state stay non-temporal: plain ones +-1%): with
+//   265,484 float32 Adam parameters and the gradient kept, 6 / 8 / 12 / 16 / 20
+//   replicas +5% / +11% / +11% / +12% / +7%, but 3-4 replicas (16-21 MB) -4% to
+//   0, 25 MB without the gradient -4%, and 28-100 (148 MB on) -8%.
+//   1: the store of the consolidated gradient, which nothing here reads again,
+//   for gradients up to kSegCacheGrad: 28 / 32 / 48 / 64 / 80 replicas +3% / +5%
+//   / +7% / +7% / +9%, 32 x 545,100 SGD +6%, but 102 MB -2%, 140 MB and more -3%
+//   to -4%, and under kSegCacheMin -3%.
+// A branch on the launch's kind inside one kernel lost up to 6% of the gain.
+constexpr int64_t kSegCacheMin = int64_t(27) << 20;
+constexpr int64_t kSegCacheGrad = int64_t(88) << 20;
+
 // PRE: the per-replica constants come from the call's workspace (a.k.vec.pre).
-template <typename P, bool ANY, bool PRE>
+// CACHE: plain accesses to the gradient buffer (1) and for every load (2).
+template <typename P, bool ANY, bool PRE, int CACHE = 0>
 __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(SegArgs<P> a) {
+  constexpr bool NTG = CACHE == 0, NTL = CACHE < 2;
   using T = typename P::T;
   using S = typename P::S;
   constexpr int NS = P::NS;
@@ -2248,14 +2284,14 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
   Packs<ANY, S, true, KP> sp[SS];
 #pragma unroll
   for (int b = 0; b < NS; ++b) sp[b] = Packs<ANY, S, true, KP>(srow[b] + t.first);
-  const Packs<ANY, T, true, KP> gout(g_dst != nullptr ? g_dst + t.first : nullptr);
+  const Packs<ANY, T, NTG, KP> gout(g_dst != nullptr ? g_dst + t.first : nullptr);
   Pack<T, KP> vp[U], vg[U];
   Pack<S, KP> vs[SS][U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t i = int64_t(u) * NTH + threadIdx.x;
     if (i < t.packs) {
-      vp[u] = load_stream(pp + i);
+      vp[u] = load_stream<NTL>(pp + i);
       if (gap) {
         if (g_src != nullptr) {
           vg[u] = gout.load(i);  // a gap reads the consolidated gradient
@@ -2264,11 +2300,13 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
           for (int k = 0; k < KP; ++k) vg[u].v[k] = zero;
         }
       } else {
-        vg[u] = load_stream_any<true, KP>(g_src + t.first + i * KP);
+        vg[u] = load_stream_any<NTL, KP>(g_src + t.first + i * KP);
       }
       if (load_state) {
 #pragma unroll
-        for (int b = 0; b < NS; ++b) vs[b][u] = sp[b].load(i);
+        for (int b = 0; b < NS; ++b) {
+          vs[b][u] = Packs<ANY, S, NTL, KP>(srow[b] + t.first).load(i);
+        }
       }
     }
   }
@@ -2881,7 +2919,8 @@ int launch_dense(const Call& c, int nbufs) {
   // workspace where the policy has one, and for SGD, which has none.
   const bool small =
       (pre || P::kPreWords == 0) &&
-      c.R <= P::kStreamSmallBytes / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1);
+      c.R <= kMallBytes / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1) &&
+      c.R * c.T * operand_bytes_per_elem<P>() >= P::kStreamSmallFrom;
   const bool mid =
       c.R <= kMidBytes / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1);
   const auto prepare = [&] {
@@ -2962,6 +3001,7 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
   if (n_segs < 0 || (n_segs > 0 && segs == nullptr)) return kInvalid;
   SegArgs<P> a;
   bool vec_rows = false;
+  int cache = 0;
   const SegmentWalk walk{segs, n_segs, c.T, true};
   const bool pre = uses_workspace<P>(c);
   const int64_t tile = pre ? segment_tile<P, true>() : segment_tile<P, false>();
@@ -2973,6 +3013,14 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
     vec_rows = rows_streamable<P>(a.k.x, nbufs, a.k.g.res0, a.k.g.rmod);
     const int nth = pre ? segment_threads<P, true>() : segment_threads<P, false>();
     if (!walk_fits(walk, c.R, tile, nth)) return false;
+    const int64_t elems = c.R * c.T;
+    const bool keeps = a.k.x.data[1] != nullptr;
+    const int64_t bytes = elems * (operand_bytes_per_elem<P>() + (keeps ? sizeof(T) : 0));
+    if (bytes >= kSegCacheMin) {
+      cache = bytes <= kMallBytes                                        ? 2
+              : keeps && elems * int64_t(sizeof(T)) <= kSegCacheGrad ? 1
+                                                                     : 0;
+    }
     // No more workgroups than this, heads included: T / tile, the last tile of
     // every segment and of every gap, and one head, per replica.
     const uint64_t most = static_cast<uint64_t>(c.R) * (c.T / tile + 2 * n_segs + 3);
@@ -2984,6 +3032,13 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
     uint32_t* const heads = &a.k.g.heads;
     const bool same_phase =
         rows_same_phase<P>(a.k.x, nbufs, stream_pack<typename P::T, typename P::S>());
+    const auto launch = [&](auto kernel, uint32_t lds, int nth) {
+      return launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg, kernel, c.stream, lds, nth,
+                            heads);
+    };
+    // The forms the operators run (with a workspace where the policy has one)
+    // come with plain accesses too, for operands that share a phase.
+    constexpr bool kCached = P::kPreWords == 0;
     if constexpr (P::kPreWords > 0) {
       if (pre) {
         constexpr int nth = segment_threads<P, true>();
@@ -2991,17 +3046,19 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
         // launches: at least kCapMinElems elements)
         const uint32_t lds =
             c.R * c.T >= kCapMinElems ? segment_lds_pre_of<P>::value : 0u;
-        return same_phase ? launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg,
-                                           segment_kernel<P, false, true>, c.stream, lds, nth, heads)
-                          : launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg,
-                                           segment_kernel<P, true, true>, c.stream, lds, nth, heads);
+        if (!same_phase) return launch(segment_kernel<P, true, true>, lds, nth);
+        if (cache == 2) return launch(segment_kernel<P, false, true, 2>, lds, nth);
+        if (cache == 1) return launch(segment_kernel<P, false, true, 1>, lds, nth);
+        return launch(segment_kernel<P, false, true>, lds, nth);
       }
     }
     constexpr int nth = segment_threads<P, false>();
-    return same_phase ? launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg,
-                                       segment_kernel<P, false, false>, c.stream, 0, nth, heads)
-                      : launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg,
-                                       segment_kernel<P, true, false>, c.stream, 0, nth, heads);
+    if (!same_phase) return launch(segment_kernel<P, true, false>, 0, nth);
+    if constexpr (kCached) {
+      if (cache == 2) return launch(segment_kernel<P, false, false, 2>, 0, nth);
+      if (cache == 1) return launch(segment_kernel<P, false, false, 1>, 0, nth);
+    }
+    return launch(segment_kernel<P, false, false>, 0, nth);
   });
 }
 
