@@ -40,8 +40,10 @@
 
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
+#include <c10/core/Allocator.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/util/SmallVector.h>
 #include <torch/library.h>
 
 #include <algorithm>
@@ -154,17 +156,18 @@ struct Prepared {
   uint32_t flags;
   at::Tensor steps;
   at::Tensor mask;
-  std::vector<at::Tensor> hyp;
+  c10::SmallVector<at::Tensor, 5> hyp;
   at::Tensor out;
-  at::Tensor ws;
+  c10::DataPtr ws;
+  size_t ws_size = 0;
   int64_t R, T;
   hipStream_t stream;
 
   const void* h(size_t i) const { return hyp[i].data_ptr(); }
   const uint8_t* m() const { return static_cast<const uint8_t*>(mask.data_ptr()); }
-  bool has_ws() const { return ws.defined(); }
-  void* ws_ptr() const { return ws.data_ptr(); }
-  size_t ws_bytes() const { return static_cast<size_t>(ws.numel()); }
+  bool has_ws() const { return ws_size > 0; }
+  void* ws_ptr() const { return ws.get(); }
+  size_t ws_bytes() const { return ws_size; }
 };
 
 Prepared prepare(const at::Tensor& params, at::Tensor& state_steps,
@@ -195,11 +198,10 @@ Prepared prepare(const at::Tensor& params, at::Tensor& state_steps,
   p.out = at::empty({}, params.options());
   p.R = params.size(0);
   p.T = params.size(1);
-  size_t bytes = p.T > 0 ? ts_single_launch_bytes(p.R) : 0;
-  if (bytes == 0 && has_constants && p.T > 0) bytes = ts_workspace_bytes(p.R);
-  if (bytes > 0) {
-    p.ws = at::empty({static_cast<int64_t>(bytes)}, params.options().dtype(at::kByte));
-  }
+  p.ws_size = p.T > 0 ? ts_single_launch_bytes(p.R) : 0;
+  if (p.ws_size == 0 && has_constants && p.T > 0) p.ws_size = ts_workspace_bytes(p.R);
+  // The allocator itself: a byte tensor around it took 1.5 us more of the host.
+  if (p.ws_size > 0) p.ws = c10::GetAllocator(params.device().type())->allocate(p.ws_size);
   p.stream = current_stream(params);
   return p;
 }
@@ -214,16 +216,20 @@ struct SegTable {
 
 // Each gradient is (R, *shape) and stands for columns [col, col + numel) of
 // params; the table is returned in ascending column order, checked in range
-// and non-overlapping.
+// and non-overlapping. A contiguous gradient is read where it lies; others (and
+// all of them under `want_views`) get an (R, numel) view or copy in `keep`.
 SegTable segments_of(const at::Tensor& params, at::TensorList grads, at::IntArrayRef cols,
-                     const char* op) {
+                     const char* op, bool want_views = false) {
   TORCH_CHECK(grads.size() == cols.size(), op, ": got ", grads.size(), " gradients but ",
               cols.size(), " column offsets");
   const int64_t R = params.size(0), T = params.size(1);
-  std::vector<size_t> order(grads.size());
+  c10::SmallVector<size_t, 64> order(grads.size());
   std::iota(order.begin(), order.end(), 0);
-  std::sort(order.begin(), order.end(), [&](size_t a, size_t b) { return cols[a] < cols[b]; });
+  if (!std::is_sorted(cols.begin(), cols.end())) {
+    std::sort(order.begin(), order.end(), [&](size_t a, size_t b) { return cols[a] < cols[b]; });
+  }
   SegTable st;
+  st.segs.reserve(grads.size());
   int64_t end = 0;
   for (size_t i : order) {
     const at::Tensor& g = grads[i];
@@ -240,6 +246,10 @@ SegTable segments_of(const at::Tensor& params, at::TensorList grads, at::IntArra
     TORCH_CHECK(cols[i] >= end, op, ": gradient ", i, " (columns ", cols[i], "..",
                 cols[i] + numel, ") overlaps another gradient");
     end = cols[i] + numel;
+    if (g.is_contiguous() && !want_views) {
+      st.segs.push_back(ts_segment{g.data_ptr(), numel, cols[i], numel});
+      continue;
+    }
     at::Tensor g2 = g.reshape({R, numel});
     if (g2.stride(1) != 1) g2 = g2.contiguous();
     st.segs.push_back(ts_segment{g2.data_ptr(), g2.stride(0), cols[i], numel});
@@ -504,7 +514,7 @@ at::Tensor adagrad_step_segments_gpu(at::Tensor params, at::TensorList grads,
 void scatter_grads_cpu(at::Tensor dst, at::TensorList grads, at::IntArrayRef cols) {
   constexpr const char* op = "churten::scatter_grads_";
   TORCH_CHECK(dst.dim() == 2, op, ": dst must be a 2-D (R, T) buffer");
-  const SegTable st = segments_of(dst, grads, cols, op);
+  const SegTable st = segments_of(dst, grads, cols, op, /*want_views=*/true);
   for (size_t i = 0; i < st.segs.size(); ++i) {
     dst.narrow(1, st.segs[i].col, st.segs[i].numel).copy_(st.keep[i]);
   }

@@ -21,7 +21,7 @@ def lead_squeeze(t: torch.Tensor, d: int | None) -> torch.Tensor:
     """Batch dim to the front, then drop a singleton replica dim behind it."""
     if d is None:
         return t
-    out = torch.movedim(t, d, 0)
+    out = t if d == 0 else torch.movedim(t, d, 0)
     if out.dim() >= 2 and out.size(1) == 1:
         out = out.squeeze(1)
     return out

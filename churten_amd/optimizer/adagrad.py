@@ -14,7 +14,7 @@ import torch
 from churten_amd.kernels.adagrad import adagrad_step_, adagrad_step_f32_
 from churten_amd.kernels.segments import adagrad_step_segments_
 from churten_amd.optimizer.grad_transform import GradientTransformation
-from churten_amd.state import State
+from churten_amd.state import State, as_rows, as_vector
 
 __all__ = ["Adagrad", "adagrad_step_"]
 
@@ -45,13 +45,13 @@ class Adagrad(metaclass=GradientTransformation):
     def _state_args(cls, state: State, maximize=False):
         opt = state.optimizer_state
         args = (
-            torch.atleast_2d(opt["state_sums"]),
-            torch.atleast_1d(opt["state_steps"]),
-            torch.atleast_1d(opt["lr"]),
-            torch.atleast_1d(opt["lr_decay"]),
-            torch.atleast_1d(opt["weight_decay"]),
-            torch.atleast_1d(opt["eps"]),
-            torch.atleast_1d(state.active_mask),
+            as_rows(opt["state_sums"]),
+            as_vector(opt["state_steps"]),
+            as_vector(opt["lr"]),
+            as_vector(opt["lr_decay"]),
+            as_vector(opt["weight_decay"]),
+            as_vector(opt["eps"]),
+            as_vector(state.active_mask),
         )
         return args, dict(maximize=bool(opt.get("maximize", maximize)))
 
@@ -59,7 +59,7 @@ class Adagrad(metaclass=GradientTransformation):
     def update(cls, state: State, maximize: bool = False) -> State:
         args, flags = cls._state_args(state, maximize)
         op = adagrad_step_f32_ if state.optimizer_state.get("fp32_math") else adagrad_step_
-        op(torch.atleast_2d(state.flat_params), torch.atleast_2d(state.flat_grads), *args,
+        op(as_rows(state.flat_params), as_rows(state.flat_grads), *args,
            **flags)
         return state
 
@@ -69,7 +69,7 @@ class Adagrad(metaclass=GradientTransformation):
         (``churten::adagrad_step_segments_``); ``grads_out`` receives the
         consolidated gradient unless it is None."""
         args, flags = cls._state_args(state)
-        adagrad_step_segments_(torch.atleast_2d(state.flat_params), grads, cols, grads_out,
+        adagrad_step_segments_(as_rows(state.flat_params), grads, cols, grads_out,
                                *args, fp32_math=bool(state.optimizer_state.get("fp32_math")),
                                **flags)
         return state

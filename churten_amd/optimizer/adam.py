@@ -17,7 +17,7 @@ import torch
 from churten_amd.kernels.adam import adam_step_
 from churten_amd.kernels.segments import adam_step_segments_
 from churten_amd.optimizer.grad_transform import GradientTransformation
-from churten_amd.state import State
+from churten_amd.state import State, as_rows, as_vector
 
 __all__ = ["Adam", "adam_step_"]
 
@@ -48,16 +48,16 @@ class Adam(metaclass=GradientTransformation):
         opt = state.optimizer_state
         mx = opt.get("max_exp_avg_sqs")
         args = (
-            torch.atleast_2d(opt["exp_avgs"]),
-            torch.atleast_2d(opt["exp_avg_sqs"]),
-            torch.atleast_2d(mx) if mx is not None else None,
-            torch.atleast_1d(opt["state_steps"]),
-            torch.atleast_1d(opt["lr"]),
-            torch.atleast_1d(opt["beta1"]),
-            torch.atleast_1d(opt["beta2"]),
-            torch.atleast_1d(opt["eps"]),
-            torch.atleast_1d(opt["weight_decay"]),
-            torch.atleast_1d(state.active_mask),
+            as_rows(opt["exp_avgs"]),
+            as_rows(opt["exp_avg_sqs"]),
+            as_rows(mx) if mx is not None else None,
+            as_vector(opt["state_steps"]),
+            as_vector(opt["lr"]),
+            as_vector(opt["beta1"]),
+            as_vector(opt["beta2"]),
+            as_vector(opt["eps"]),
+            as_vector(opt["weight_decay"]),
+            as_vector(state.active_mask),
         )
         flags = dict(
             amsgrad=bool(opt.get("amsgrad", amsgrad)),
@@ -71,7 +71,7 @@ class Adam(metaclass=GradientTransformation):
     def update(cls, state: State, decoupled_weight_decay: bool = True, maximize: bool = False,
                amsgrad: bool = False) -> State:
         args, flags = cls._state_args(state, decoupled_weight_decay, maximize, amsgrad)
-        adam_step_(torch.atleast_2d(state.flat_params), torch.atleast_2d(state.flat_grads),
+        adam_step_(as_rows(state.flat_params), as_rows(state.flat_grads),
                    *args, **flags)
         return state
 
@@ -81,6 +81,6 @@ class Adam(metaclass=GradientTransformation):
         (``churten::adam_step_segments_``); ``grads_out`` receives the
         consolidated gradient unless it is None."""
         args, flags = cls._state_args(state)
-        adam_step_segments_(torch.atleast_2d(state.flat_params), grads, cols, grads_out,
+        adam_step_segments_(as_rows(state.flat_params), grads, cols, grads_out,
                             *args, **flags)
         return state

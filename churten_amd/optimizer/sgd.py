@@ -17,7 +17,7 @@ import torch
 from churten_amd.kernels.segments import sgd_step_segments_
 from churten_amd.kernels.sgd import sgd_step_
 from churten_amd.optimizer.grad_transform import GradientTransformation
-from churten_amd.state import State
+from churten_amd.state import State, as_rows, as_vector
 
 __all__ = ["SGD", "sgd_step_"]
 
@@ -51,21 +51,21 @@ class SGD(metaclass=GradientTransformation):
         opt = state.optimizer_state
         mb = opt.get("momentum_buffers")
         args = (
-            torch.atleast_1d(opt["state_steps"]),
-            torch.atleast_1d(opt["lr"]),
-            torch.atleast_1d(opt["momentum"]),
-            torch.atleast_1d(opt["dampening"]),
-            torch.atleast_1d(opt["weight_decay"]),
-            torch.atleast_1d(state.active_mask),
+            as_vector(opt["state_steps"]),
+            as_vector(opt["lr"]),
+            as_vector(opt["momentum"]),
+            as_vector(opt["dampening"]),
+            as_vector(opt["weight_decay"]),
+            as_vector(state.active_mask),
         )
         flags = dict(nesterov=bool(opt.get("nesterov", nesterov)),
                      maximize=bool(opt.get("maximize", maximize)))
-        return torch.atleast_2d(mb) if mb is not None else None, args, flags
+        return as_rows(mb) if mb is not None else None, args, flags
 
     @classmethod
     def update(cls, state: State, nesterov: bool = False, maximize: bool = False) -> State:
         mb, args, flags = cls._state_args(state, nesterov, maximize)
-        sgd_step_(torch.atleast_2d(state.flat_params), torch.atleast_2d(state.flat_grads), mb,
+        sgd_step_(as_rows(state.flat_params), as_rows(state.flat_grads), mb,
                   *args, **flags)
         return state
 
@@ -75,6 +75,6 @@ class SGD(metaclass=GradientTransformation):
         (``churten::sgd_step_segments_``); ``grads_out`` receives the
         consolidated gradient unless it is None."""
         mb, args, flags = cls._state_args(state)
-        sgd_step_segments_(torch.atleast_2d(state.flat_params), grads, cols, grads_out, mb,
+        sgd_step_segments_(as_rows(state.flat_params), grads, cols, grads_out, mb,
                            *args, **flags)
         return state

@@ -1,0 +1,94 @@
+"""The gradient table apply_gradient builds from a per-name dict: what goes to
+the fused path, what falls back to the per-name copies, and that every layout a
+gradient can have ends up in the same columns (CPU key)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import churten_amd.kernels  # noqa: F401
+from churten_amd.optimizer import SGD
+from churten_amd.state import State
+
+SHAPES = {"a": (3, 2), "b": (3,), "c": (2, 3, 2), "d": ()}
+
+
+def make(meta_type=torch.Size, dtype=torch.float32):
+    meta, off = [], 0
+    for name, s in SHAPES.items():
+        n = int(torch.Size(s).numel())
+        meta.append((name, meta_type((4, *s)), off, n))
+        off += n
+    T = off + (-off % 4)
+    p = torch.arange(4 * T, dtype=dtype).reshape(4, T)
+    state = State(params=p, buffers=torch.empty(4, 0), param_meta=meta, buffer_meta=[])
+    return SGD.init(state, lr=0.5)
+
+
+def grads_of(dtype=torch.float32):
+    g = torch.Generator().manual_seed(4)
+    return {k: torch.randn(4, *s, generator=g).to(dtype) for k, s in SHAPES.items()}
+
+
+def consolidated(grads, T):
+    out = torch.zeros(4, T)
+    off = 0
+    for k, s in SHAPES.items():
+        n = int(torch.Size(s).numel())
+        out[:, off:off + n] = grads[k].detach().reshape(4, n)
+        off += n
+    return out
+
+
+def strided(t):
+    wide = torch.zeros(*t.shape[:-1], 2 * t.shape[-1])
+    wide[..., ::2] = t
+    return wide[..., ::2]
+
+
+LAYOUTS = {
+    "contiguous": lambda k, t: t,
+    "requires_grad": lambda k, t: t.clone().requires_grad_(),
+    "row_strided": lambda k, t: torch.cat([t[:, None], t[:, None]], dim=1)[:, 0],
+    "inner_strided": lambda k, t: strided(t) if t.dim() > 1 else t,
+    "transposed": lambda k, t: t.transpose(0, -1).contiguous().transpose(0, -1),
+    "expanded": lambda k, t: t[:1].expand(t.shape),
+}
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("order", [1, -1])
+@pytest.mark.parametrize("meta_type", [torch.Size, list, tuple])
+def test_layouts(layout, order, meta_type):
+    state = make(meta_type)
+    grads = {k: LAYOUTS[layout](k, t) for k, t in list(grads_of().items())[::order]}
+    before = state.params.clone()
+    want = consolidated(grads, state.params.shape[1])
+    SGD.apply_gradient(state, grads)
+    assert torch.equal(state.grads, want)
+    assert torch.equal(state.params, before - 0.5 * want)
+
+
+def test_what_falls_back():
+    state = make()
+    table = state._consolidated_grads.segments
+    full = grads_of()
+    assert table(full)[1] == [0, 6, 9, 21]
+    assert table({"c": full["c"]})[1] == [9]  # part of the names
+    assert table({}) == ([], [])
+    for bad in ({"zz": full["a"]}, {"a": full["a"], "zz": full["b"]}, {"a": None},
+                {"a": full["a"].double()}, {"a": full["a"][:3]}, {"a": full["a"][0]},
+                {"a": full["a"].reshape(4, 6)}, {"a": 1.0}):
+        assert table(bad) is None
+
+
+def test_unknown_name_is_refused_and_views_still_alias():
+    state = make()
+    grads = grads_of()
+    with pytest.raises(KeyError):
+        SGD.apply_gradient(state, {**{k: grads[k] for k in "abc"}, "zz": grads["d"]})
+    view = state._consolidated_grads
+    assert list(view.keys()) == list(SHAPES)
+    view["b"].fill_(2.0)
+    assert bool((state.grads[:, 6:9] == 2.0).all())
