@@ -685,6 +685,14 @@ struct AdamPolicy {
   // scalar too.
   static constexpr bool kSegmentScalarMask = true;
   static constexpr uint32_t kSegmentLdsPre = kFp32State<T, S> ? lds_for_residency(20) : 0u;
+  // Above kMidBytes of operands fewer still: 12 where the gradient is kept, 14
+  // where it is not. With the loads issued before the constants, whole calls
+  // against a cap of 20, same process, kept / not: 1.9 GB +1.0% / +0.7%, 3.1 GB
+  // +1.3% / +1.0%, 3.8 GB +1.8% / +1.6% (8 rows; 32 shorter ones -0.9% / +0.2%),
+  // 12 GB +5.0% / +2.9%, 15 GB +2.7% / +2.5%; at 0.36-1.0 GB 12 loses 1-5% and 14
+  // moves -1.5% to +0.9%.
+  static constexpr uint32_t kSegmentLdsKept = kFp32State<T, S> ? lds_for_residency(12) : 0u;
+  static constexpr uint32_t kSegmentLdsFused = kFp32State<T, S> ? lds_for_residency(14) : 0u;
   static constexpr bool kLateStores = !AMSGRAD && std::is_same<T_, float>::value;
   static constexpr bool kVariant = false;
   static constexpr int kPreWords = 2;
@@ -1207,6 +1215,24 @@ template <typename P>
 struct segment_lds_pre_of<P, std::void_t<decltype(P::kSegmentLdsPre)>> {
   static constexpr uint32_t value = P::kSegmentLdsPre;
 };
+// The reservation of a segmented launch with a workspace: `large` beyond
+// kMidBytes of operands, `kept` with the consolidated gradient written.
+template <typename P, typename = void>
+struct segment_lds_large_of {
+  static constexpr uint32_t kept = segment_lds_pre_of<P>::value;
+  static constexpr uint32_t fused = kept;
+};
+template <typename P>
+struct segment_lds_large_of<P, std::void_t<decltype(P::kSegmentLdsKept)>> {
+  static constexpr uint32_t kept = P::kSegmentLdsKept;
+  static constexpr uint32_t fused = P::kSegmentLdsFused;
+};
+template <typename P>
+uint32_t segment_lds(bool large, bool kept) {
+  return !large ? segment_lds_pre_of<P>::value
+         : kept ? segment_lds_large_of<P>::kept
+                : segment_lds_large_of<P>::fused;
+}
 
 // Replica r's active flag through the scalar cache: one s_load_dword of the
 // aligned dword that holds byte r (that dword never leaves the page the byte
@@ -3002,6 +3028,7 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
   SegArgs<P> a;
   bool vec_rows = false;
   int cache = 0;
+  bool large = false;
   const SegmentWalk walk{segs, n_segs, c.T, true};
   const bool pre = uses_workspace<P>(c);
   const int64_t tile = pre ? segment_tile<P, true>() : segment_tile<P, false>();
@@ -3016,6 +3043,7 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
     const int64_t elems = c.R * c.T;
     const bool keeps = a.k.x.data[1] != nullptr;
     const int64_t bytes = elems * (operand_bytes_per_elem<P>() + (keeps ? sizeof(T) : 0));
+    large = bytes > kMidBytes;
     if (bytes >= kSegCacheMin) {
       cache = bytes <= kMallBytes                                        ? 2
               : keeps && elems * int64_t(sizeof(T)) <= kSegCacheGrad ? 1
@@ -3044,8 +3072,9 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
         constexpr int nth = segment_threads<P, true>();
         // the cap only where it can pay (as for the streaming driver's
         // launches: at least kCapMinElems elements)
-        const uint32_t lds =
-            c.R * c.T >= kCapMinElems ? segment_lds_pre_of<P>::value : 0u;
+        const uint32_t lds = c.R * c.T >= kCapMinElems
+                                 ? segment_lds<P>(large, a.k.x.data[1] != nullptr)
+                                 : 0u;
         if (!same_phase) return launch(segment_kernel<P, true, true>, lds, nth);
         if (cache == 2) return launch(segment_kernel<P, false, true, 2>, lds, nth);
         if (cache == 1) return launch(segment_kernel<P, false, true, 1>, lds, nth);
