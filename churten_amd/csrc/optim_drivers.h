@@ -658,8 +658,12 @@ struct AdamPolicy {
   // the flag read through the scalar cache (same-process A/B at config 1's
   // shape, 200 calls x 4 rounds: float16 / bfloat16 params +27% / +32%,
   // bfloat16 moments +19% against four packs with the vector read; two packs
-  // +10-18%; the scalar read alone +-0.6%). float64 kept its two packs (+-1%).
-  static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(2, 1, 1, 2);
+  // +10-18%; the scalar read alone +-0.6%). float32 and float64 moved from two
+  // packs to one when the call became a single launch (whole calls, same
+  // process: 34 / 51 / 68 / 85 MB of float32 operands +5% / +4% / +2% / +5%, with
+  // amsgrad -1% to +6%, float64 -3% to +16%; 128 and 256 threads 4-8% slower, the
+  // scalar read +-1%).
+  static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 1, 1);
   static constexpr bool kScalarMaskSmall =
       !kFp32State<T, S> && !std::is_same<T, double>::value;
   static constexpr int64_t kStreamSmallFrom =
@@ -796,7 +800,7 @@ struct SgdPolicy {
   static constexpr uint32_t kStreamLdsPre = kStreamLds;
   static constexpr uint32_t kStreamLdsMid = kStreamLdsPre;
   static constexpr int kStreamUnrollPre = kStreamUnroll;
-  static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 4, 2);
+  static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 4, 1);
   static constexpr bool kScalarMask =
       std::is_same<T, float>::value || (HAS_BUF && std::is_same<T, double>::value);
   static constexpr bool kScalarMaskSmall = kScalarMask;
@@ -887,7 +891,9 @@ struct AdagradPolicy {
   // MALL-resident 16-bit launches: one pack, the scalar flag read (at config
   // 4's shape against four packs with the vector read: bfloat16 +12%, float16
   // +9%; two packs +5%).
-  static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(2, 1, 1, 2);
+  // float32 and float64: one pack too in a single launch (two: -2% to -12% at
+  // 19-97 MB).
+  static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 1, 1);
   static constexpr bool kScalarMaskSmall = sizeof(T) == 2;
   static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
   static constexpr int kStreamPack = stream_pack<T, S>();
@@ -1012,7 +1018,8 @@ struct AdagradF32Policy {
   static constexpr uint32_t kStreamLdsMid = kStreamLdsPre;
   static constexpr int kStreamUnrollPre = stream_unroll<T, S>(1, 1, 1, 2);
   static constexpr bool kScalarMask = std::is_same<T, float>::value;
-  static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(2, 1, 4, 2);
+  // float32: one pack in a single launch (two: -1% to -17% at 19-97 MB).
+  static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 4, 1);
   static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
   static constexpr int kStreamPack = stream_pack<T, S>();
   // Segmented with a workspace: one-wavefront workgroups, one pack, the
