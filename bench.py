@@ -426,7 +426,7 @@ def size_sweep_timing(cfg: int, ns, launches: int):
     """The config's update on the first n rows of one allocation of max(ns)
     rows (same buffers, same per-replica hyperparameters and mask, so only
     the size changes), kernel-only time per launch, and per launch-size class
-    (operands up to 256 MB: small, up to 1 GiB: mid, above: large; each class
+    (operands up to 100 MiB: small, up to 1 GiB: mid, above: large; each class
     has its own launch shape) a least-squares fit t = t0 + bytes / rate: t0 is
     what a launch costs beyond streaming its bytes (the preparation launch,
     the grid's ramp-up, the drain of its last workgroups), `rate` the
@@ -445,7 +445,7 @@ def size_sweep_timing(cfg: int, ns, launches: int):
         ms = kernel_only_timing(op_name, args, kw, launches)
         opb = n * T * 4 * n_rt
         pts.append({"N": n, "active": active, "bytes": nbytes, "operand_bytes": opb,
-                    "class": "small" if opb <= 256 << 20 else "mid" if opb <= 1 << 30 else "large",
+                    "class": "small" if opb <= 100 << 20 else "mid" if opb <= 1 << 30 else "large",
                     "kernel_avg_us": round(ms * 1e3, 2),
                     "GBs": round(nbytes / (ms * 1e-3) / 1e9, 1)})
     del full, args
@@ -1146,9 +1146,10 @@ def main():
                   "true" if op_args[2] is not None else "false", str(kw.get("nesterov")).lower()),
               "adagrad": "AdagradPolicy<float, float>"}[op_name]
     # the instantiation the operator launches: ANY = false (State's layout), PRE (per-replica
-    # constants from the workspace: Adam and Adagrad), SMALL (operands that fit the 256 MB MALL)
+    # constants from the workspace: Adam and Adagrad), SMALL (operands of up to 100 MiB,
+    # which the MALL keeps between steps)
     n_rt = sum(t is not None and t.dim() == 2 for t in op_args)
-    small = op_args[0].numel() * 4 * n_rt <= 256 << 20
+    small = op_args[0].numel() * 4 * n_rt <= 100 << 20
     kernel = "stream_kernel<%s, false, %s, %s>" % (policy, str(op_name != "sgd").lower(),
                                                   str(small).lower())
     profile_key = f"{op_name}_stream_kernel_cfg{args.config}"
