@@ -136,7 +136,7 @@ using PackBits = uint32_t __attribute__((ext_vector_type(sizeof(T) * N / 4)));
 
 // Streaming accesses: every byte of the optimizer state is touched exactly
 // once per step, so the loads and stores carry the non-temporal hint (NT).
-// Launches whose operands fit the 256 MB MALL several times over take plain,
+// Launches whose operands the 256 MB MALL keeps between steps take plain,
 // cache-allocating accesses instead (NT = false): back-to-back steps then hit
 // the MALL (see the streaming driver's launch).
 template <bool NT, typename V>
@@ -411,7 +411,7 @@ __device__ __forceinline__ double wave_lane(double x, int lane) {
 // each policy's reservations; small launches (under kCapMinElems elements of
 // the (R, T) operands, 8192 tiles of 512) launch without them, since there the
 // cap would only serialise the launch (config 1 lost 16% with one). The
-// segmented driver runs uncapped (its shapes are next to segment_tile).
+// segmented driver has caps of its own (kSegmentLds*, next to segment_tile).
 constexpr uint32_t kLdsPerCU = 160 * 1024;
 constexpr uint32_t lds_for_residency(uint32_t n) {
   uint32_t x = (kLdsPerCU / n) / 256 * 256;
@@ -662,7 +662,9 @@ struct AdamPolicy {
   // packs to one when the call became a single launch (whole calls, same
   // process: 34 / 51 / 68 / 85 MB of float32 operands +5% / +4% / +2% / +5%, with
   // amsgrad -1% to +6%, float64 -3% to +16%; 128 and 256 threads 4-8% slower, the
-  // scalar read +-1%).
+  // scalar read +-1%). With a preparation launch in front (a capture, a smaller
+  // workspace) two packs had been 6% ahead at 34 MB; the shape follows the form
+  // that the operators run.
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 1, 1);
   static constexpr bool kScalarMaskSmall =
       !kFp32State<T, S> && !std::is_same<T, double>::value;
