@@ -531,7 +531,8 @@ constexpr int stream_unroll(int fp32, int bf16_state, int narrow, int wide) {
 // two-launch calls never read a workspace). `reads_state` is decided from the
 // (R,) vectors alone, so the drivers issue their loads before the constants;
 // `may_read_state` and `needs_entry` are its like in a single launch, where the
-// step may be seen from before or after the bump.
+// step may be seen from before or after the bump (`kSkipsState`: the first may
+// turn out wrong once the constants are there, as `skips_state` then says).
 // `decays` / `drop_decay`: whether the replica's weight-decay term is live, and
 // a copy of its constants with the decay set to a literal zero (the element
 // math then skips the term, exactly as it does for a zero decay at run time).
@@ -758,8 +759,9 @@ struct AdamPolicy {
     rep.h.weight_decay = hyper_at(v.h[4], r);
   }
   __device__ static bool reads_state(const Vectors<T>&, uint32_t) { return true; }
-  __device__ static bool may_read_state(T, bool) { return true; }
-  __device__ static bool needs_entry(T, bool) { return true; }
+  static constexpr bool kSkipsState = false;
+  __device__ static bool may_read_state(T, T) { return true; }
+  __device__ static bool needs_entry(T, T) { return true; }
   __device__ static bool decays(const Rep& rep) { return rep.h.weight_decay != 0; }
   __device__ static void drop_decay(Rep& rep) { rep.h.weight_decay = 0.0; }
   __device__ static void update(M& p, M g, M (&s)[NS], const Rep& rep, bool maximize) {
@@ -854,11 +856,19 @@ struct SgdPolicy {
   __device__ static bool reads_state(const Vectors<T>& v, uint32_t r) {
     return widen(v.steps[r]) != M(1);
   }
-  // The same from a step read while it may be bumped: 0 is from before a first
-  // step's bump, and only 1 needs the entry (a first step's new step, or the
-  // old one of the second).
-  __device__ static bool may_read_state(T x, bool bump) { return widen(x) != M(bump ? 0 : 1); }
-  __device__ static bool needs_entry(T x, bool bump) { return bump && widen(x) == M(1); }
+  // The same where the step is read while it may be bumped: `x` is the old step
+  // or the new one, `next` is what a bump makes of x. A new step is 1 on a first
+  // step only, so where `next` is 1 the buffer is taken for unread (x is most
+  // likely the old step), and where x or `next` is 1 the entry decides: x = 1 is
+  // a first step's new one or the second's old one, x = 0 a first step's old one
+  // or the new one of a counter that stood at -1. A buffer that was taken for
+  // unread wrongly is fetched after the constants (skips_state).
+  static constexpr bool kSkipsState = HAS_BUF;
+  __device__ static bool skips_state(const Rep& rep) { return rep.first; }
+  __device__ static bool may_read_state(T, T next) { return widen(next) != M(1); }
+  __device__ static bool needs_entry(T x, T next) {
+    return widen(x) != widen(next) && (widen(x) == M(1) || widen(next) == M(1));
+  }
   __device__ static bool decays(const Rep& rep) { return rep.h.weight_decay != 0; }
   __device__ static void drop_decay(Rep& rep) { rep.h.weight_decay = 0.0; }
   __device__ static void update(M& p, M g, M (&s)[NS > 0 ? NS : 1], const Rep& rep,
@@ -936,8 +946,9 @@ struct AdagradPolicy {
     rep.once = kVariant && ilp_row(v.ilp_rows, r);
   }
   __device__ static bool reads_state(const Vectors<T>&, uint32_t) { return true; }
-  __device__ static bool may_read_state(T, bool) { return true; }
-  __device__ static bool needs_entry(T, bool) { return true; }
+  static constexpr bool kSkipsState = false;
+  __device__ static bool may_read_state(T, T) { return true; }
+  __device__ static bool needs_entry(T, T) { return true; }
   __device__ static bool decays(const Rep& rep) { return rep.h.weight_decay != 0; }
   __device__ static void drop_decay(Rep& rep) { rep.h.weight_decay = 0.0; }
   // float16 parameters and state. torch's fused Adagrad stores the state sum
@@ -1057,8 +1068,9 @@ struct AdagradF32Policy {
     rep.h.eps = static_cast<float>(hyper_at(v.h[3], r));
   }
   __device__ static bool reads_state(const Vectors<T>&, uint32_t) { return true; }
-  __device__ static bool may_read_state(T, bool) { return true; }
-  __device__ static bool needs_entry(T, bool) { return true; }
+  static constexpr bool kSkipsState = false;
+  __device__ static bool may_read_state(T, T) { return true; }
+  __device__ static bool needs_entry(T, T) { return true; }
   __device__ static bool decays(const Rep& rep) { return rep.h.has_weight_decay; }
   __device__ static void drop_decay(Rep& rep) {
     rep.h.weight_decay = 0.0f;
@@ -1400,6 +1412,16 @@ __device__ __forceinline__ B step_is(B x) {
   }
 }
 
+// Whether the state's loads are issued before the constants are known: in a
+// single-launch call from the step as read, else from the step.
+template <typename P>
+__device__ __forceinline__ bool loads_state(const Vectors<typename P::T>& v, uint32_t r,
+                                            bool single, StepBits<typename P::T> x) {
+  if (!single) return P::reads_state(v, r);
+  const auto read = __builtin_bit_cast(typename P::T, x);
+  return P::may_read_state(read, bumped(read, v.one.bump));
+}
+
 // The constants of a replica every lane of the wavefront works on, in a
 // single-launch call. `x`: the step as read (step_read). `head`: this wavefront
 // is the replica's head and makes them known.
@@ -1412,12 +1434,12 @@ __device__ __forceinline__ void single_constants(const Vectors<typename P::T>& v
   constexpr int N = P::kConstants;
   const Single<T>& one = v.one;
   const T read = __builtin_bit_cast(T, step_is(x));
-  const bool look = !head && P::needs_entry(read, one.bump);
+  const T step = bumped(read, one.bump);
+  const bool look = !head && P::needs_entry(read, step);
   const bool late = look && blockIdx.x >= one.early;
   if (late && entry_cached(one, r, w)) return;
   const uint64_t word = look ? entry_load<N>(one, r) : 0;
   if (late && entry_is(one, word, w)) return;
-  const T step = bumped(read, one.bump);
   typename P::Rep rep;
   uniform_derive<P>(v, r, static_cast<double>(widen(step)), rep);
   P::constants(rep, w);
@@ -1694,9 +1716,7 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
   const auto run = [&](auto head_tile, int64_t first, int64_t packs_left, int64_t pre,
                        int64_t body_end) __attribute__((always_inline)) {
     const StepBits<T> x = single ? step_read(a.vec.one.steps, r) : StepBits<T>(0);
-    const bool load_state = single
-                                ? P::may_read_state(__builtin_bit_cast(T, x), a.vec.one.bump)
-                                : P::reads_state(a.vec, r);
+    bool load_state = loads_state<P>(a.vec, r, single, x);
     T* const pbase = pg_row<P>(a.x, 0, r);
     const T* const gbase = pg_row<P>(a.x, 1, r);
     S* sbase[SS];
@@ -1744,6 +1764,19 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
         call_constants<P, PRE>(a.vec, r, w);
       }
       P::set(w, rep);
+      if constexpr (P::kSkipsState) {
+        if (single && !load_state && !P::skips_state(rep)) {
+          load_state = true;
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int64_t i = int64_t(u) * NTH + threadIdx.x;
+            if (i < packs_left) {
+#pragma unroll
+              for (int b = 0; b < NS; ++b) vs[b][u] = srow[b].load(i);
+            }
+          }
+        }
+      }
     } else {
       uniform_prologue<P, PRE>(a.vec, r, rep);
     }
@@ -2261,9 +2294,7 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
 
   typename P::Rep rep;
   const StepBits<T> x = single ? step_read(a.k.vec.one.steps, r) : StepBits<T>(0);
-  const bool load_state = single
-                              ? P::may_read_state(__builtin_bit_cast(T, x), a.k.vec.one.bump)
-                              : P::reads_state(a.k.vec, r);
+  bool load_state = loads_state<P>(a.k.vec, r, single, x);
   const auto constants = [&]() __attribute__((always_inline)) {
     if constexpr (kSingle) {
       P::hypers(a.k.vec, r, rep);
@@ -2307,6 +2338,7 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
 
   if (!vec) {
     constants();
+    if constexpr (P::kSkipsState) load_state = load_state || !P::skips_state(rep);
     const int64_t cnt = imin(kSegTile, numel - j0);
     for (int64_t j = j0 + threadIdx.x; j < j0 + cnt; j += NTH) one(j);
     return;
@@ -2346,6 +2378,21 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
     }
   }
   constants();
+  if constexpr (P::kSkipsState) {
+    if (single && !load_state && !P::skips_state(rep)) {
+      load_state = true;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t i = int64_t(u) * NTH + threadIdx.x;
+        if (i < t.packs) {
+#pragma unroll
+          for (int b = 0; b < NS; ++b) {
+            vs[b][u] = Packs<ANY, S, NTL, KP>(srow[b] + t.first).load(i);
+          }
+        }
+      }
+    }
+  }
   with_variant<P>(rep, [&](const typename P::Rep& rp) {
     with_maximize<P>(a.k.maximize, [&](bool mx) {
 #pragma unroll

@@ -163,6 +163,34 @@ def test_segments(kind, kept, n_segs):
     check_same(kind, bufs, steps, mask, hyp, fill=0x5A, segs=segs)
 
 
+SGD = [KINDS[6], KINDS[7], KINDS[8], KINDS[9], ("sgd", F32, BF16, 0, 1)]
+
+
+@pytest.mark.parametrize("kind", SGD, ids=lambda k: f"{k[1]}-{k[2]}-{k[4]}")
+@pytest.mark.parametrize("n_segs", [0, 1, 70])
+@pytest.mark.parametrize("n", [3, 70001])
+def test_sgd_counters_below_zero(kind, n, n_segs):
+    """A counter may start anywhere. From -1 the new step is 0, which is also
+    the old step of a first one: the momentum buffer is read and kept there, and
+    a first step is where the *new* step is 1 (so also from a counter that a bump
+    rounds to 1). The 70 segments take two launches, the second after the bump."""
+    R, T = 9, max(n, 70 * 7 if n_segs else n)
+    bufs, steps, mask, hyp = make(kind, R, T, seed=5)
+    eps = 2.0 ** -26 if kind[1] == F32 else 2.0 ** -10 if kind[1] == BF16 else 2.0 ** -55
+    steps.copy_(torch.tensor([-1, -2, -1, 0, -0.0, -1 + 4 * eps, eps, 1, -3], dtype=F64))
+    mask[:] = True
+    mask[2] = False
+    for b in bufs[2:]:
+        b[1] = 0.5
+    segs = None
+    if n_segs:
+        g = torch.Generator(device=DEV).manual_seed(8)
+        w = T // n_segs
+        segs = [(i * w + 1, torch.randn(R, w - 2, device=DEV, generator=g).to(kind[1]))
+                for i in range(n_segs)]
+    check_same(kind, bufs, steps, mask, hyp, fill=0, calls=4, segs=segs)
+
+
 def test_replica_limit():
     assert LIB.ts_single_launch_bytes(1024) == 128 * 1024
     assert LIB.ts_single_launch_bytes(1025) == 0 and LIB.ts_single_launch_bytes(0) == 0
