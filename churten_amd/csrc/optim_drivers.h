@@ -71,8 +71,6 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <atomic>
-#include <chrono>
 #include <initializer_list>
 #include <type_traits>
 
@@ -80,6 +78,11 @@
 #include "optim_math.h"
 
 namespace churten {
+
+// A launch's identity for the entries of its workspace, from one counter for
+// the whole library (optim_kernels.hip). Not 0.
+uint64_t next_nonce();
+
 namespace {
 
 // Launch shape, measured on the MI355X over the 52 GB north-star state:
@@ -1290,7 +1293,7 @@ __device__ __forceinline__ bool mask_byte_scalar(const uint8_t* mask, uint32_t r
 // An entry holds kConstants doubles as 2 * kConstants 8-byte words, each half a
 // double next to a 32-bit tag of the launch: a word is this launch's or it is
 // not, whatever the memory held before and in whatever order the words arrive.
-// Tags do not repeat within 2^32 launches of a process (next_nonce). A call
+// An entry has both tags, and the pair is unique to the launch (next_nonce). A call
 // that is being captured into a graph, whose replays would repeat them, takes
 // two launches.
 //
@@ -2859,23 +2862,6 @@ bool fill_kargs(const Call& c, int nbufs, KArgs<P>& a, bool grad_optional) {
   a.vec.one = Single<T>{0, nullptr, nullptr, nullptr, 0, false};
   a.maximize = (c.flags & TS_MAXIMIZE) != 0;
   return true;
-}
-
-// A launch's identity for the entries of its workspace: both 32-bit halves
-// step through all their values, so neither repeats within 2^32 launches; the
-// start differs from process to process.
-inline uint64_t next_nonce() {
-  static std::atomic<uint64_t> count{
-      static_cast<uint64_t>(std::chrono::steady_clock::now().time_since_epoch().count())};
-  uint64_t nonce;
-  do {
-    const uint64_t c = count.fetch_add(1, std::memory_order_relaxed);
-    const uint32_t lo = static_cast<uint32_t>(c) * 0x9E3779B1u;
-    const uint32_t hi =
-        static_cast<uint32_t>(c) * 0x85EBCA77u + static_cast<uint32_t>(c >> 32) * 0xC2B2AE3Du;
-    nonce = uint64_t(hi) << 32 | lo;
-  } while (nonce == 0);
-  return nonce;
 }
 
 inline bool stream_capturing(hipStream_t stream) {

@@ -9,11 +9,34 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 
 #include "optim_dispatch.h"
 #include "optim_internal.h"
 
 namespace churten {
+
+// The map from the counter to the two tags is one to one (odd multipliers; the
+// low tag gives the counter's low half, the high tag then its high half), so no
+// two launches of a process share both. Each tag alone steps through all its
+// values between two changes of the high half. The counter is the library's,
+// not a translation unit's: every unit's launches meet in the same allocator's
+// blocks. Its start differs from process to process.
+uint64_t next_nonce() {
+  static std::atomic<uint64_t> count{
+      static_cast<uint64_t>(std::chrono::steady_clock::now().time_since_epoch().count())};
+  uint64_t nonce;
+  do {
+    const uint64_t c = count.fetch_add(1, std::memory_order_relaxed);
+    const uint32_t lo = static_cast<uint32_t>(c) * 0x9E3779B1u;
+    const uint32_t hi =
+        static_cast<uint32_t>(c) * 0x85EBCA77u + static_cast<uint32_t>(c >> 32) * 0xC2B2AE3Du;
+    nonce = uint64_t(hi) << 32 | lo;
+  } while (nonce == 0);
+  return nonce;
+}
+
 namespace {
 
 // Copies every segment into its columns of the (R, cols) buffer `dst`.

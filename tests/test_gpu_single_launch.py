@@ -191,6 +191,25 @@ def test_sgd_counters_below_zero(kind, n, n_segs):
     check_same(kind, bufs, steps, mask, hyp, fill=0, calls=4, segs=segs)
 
 
+def test_launches_share_one_counter():
+    """The tags of a launch come from one counter whatever entry point it went
+    through, so an entry that another optimizer's launch left is never taken for
+    this one's. They are read back from the workspaces: word i of an entry holds
+    tag i % 2 in its high half, and the low tag is the counter times an odd
+    number."""
+    odd, counts = 0x9E3779B1, []
+    for i, kind in enumerate([KINDS[0], KINDS[6], KINDS[10]] * 2):
+        for segmented in (False, True):
+            bufs, steps, mask, hyp = make(kind, 2, 64, seed=i)
+            segs = [(0, bufs[1].clone())] if segmented else None
+            ws = torch.zeros(128 * 2, device=DEV, dtype=torch.uint8)
+            call(kind, bufs, steps, mask, hyp, ws, 128 * 2, segs=segs)
+            words = ws.view(torch.int64).cpu().tolist()
+            low = (words[0] >> 32) & 0xFFFFFFFF
+            counts.append(low * pow(odd, -1, 2 ** 32) % 2 ** 32)
+    assert [(c - counts[0]) % 2 ** 32 for c in counts] == list(range(len(counts)))
+
+
 def test_replica_limit():
     assert LIB.ts_single_launch_bytes(1024) == 128 * 1024
     assert LIB.ts_single_launch_bytes(1025) == 0 and LIB.ts_single_launch_bytes(0) == 0
