@@ -24,6 +24,7 @@ optimizer-state registry. Tensordict features of the reference's class
 
 from __future__ import annotations
 
+import math
 from collections.abc import Sequence
 from functools import cached_property
 from typing import Any
@@ -97,6 +98,9 @@ def consolidated_dict_view(tcons: torch.Tensor, metadata) -> dict[str, torch.Ten
     return {name: tcons[..., off : off + n].view(*shape) for name, shape, off, n in metadata}
 
 
+_ABSENT = object()
+
+
 class _GradScatter:
     """The gradient buffer seen through per-name views; ``update_`` writes a
     per-name gradient dict into the consolidated ``(N, T)`` buffer -- in one
@@ -123,14 +127,19 @@ class _GradScatter:
     def segments(self, grads: dict[str, torch.Tensor]):
         """``(tensors, cols)`` for the fused scatter, or None when some
         gradient needs the per-name path (unknown name, other shape, dtype or
-        device)."""
-        dtype, device = self._buffer.dtype, self._buffer.device
+        device) or the metadata contradicts itself (the views refuse it)."""
+        buf = self._buffer
+        dtype, device = buf.dtype, buf.device
+        rows = buf.shape[0] if buf.ndim == 2 else math.prod(buf.shape[:-1])
         tensors, cols = [], []
-        for name, shape, off, _ in self._metadata:  # shape: the stacked (N, *shape)
-            if name not in grads:
+        for name, shape, off, n in self._metadata:  # shape: the stacked (N, *shape)
+            g = grads.get(name, _ABSENT)
+            if g is _ABSENT:
+                if math.prod(shape) != rows * n:
+                    return None
                 continue
-            g = grads[name]
             if (not isinstance(g, torch.Tensor) or g.dtype != dtype or g.device != device
+                    or g.numel() != rows * n
                     or (g.shape != shape and tuple(g.shape) != tuple(shape))):
                 return None
             tensors.append(g.detach() if g.requires_grad else g)

@@ -92,3 +92,19 @@ def test_unknown_name_is_refused_and_views_still_alias():
     assert list(view.keys()) == list(SHAPES)
     view["b"].fill_(2.0)
     assert bool((state.grads[:, 6:9] == 2.0).all())
+
+
+@pytest.mark.parametrize("bad", [("a", (4, 3, 2), 0, 5), ("b", (4, 3), 6, 4)])
+@pytest.mark.parametrize("given", ["all", "others"])
+def test_metadata_that_contradicts_itself_is_refused(bad, given):
+    """A width that is not the shape's would write the gradient's own width over
+    the next parameter's columns."""
+    state = make()
+    state.param_meta = [bad if m[0] == bad[0] else m for m in state.param_meta]
+    grads = grads_of()
+    if given == "others":
+        del grads[bad[0]]
+    before = state.params.clone()
+    with pytest.raises(RuntimeError):
+        SGD.apply_gradient(state, grads)
+    assert torch.equal(state.params, before) and not state.grads.any()
