@@ -128,6 +128,8 @@ class _GradScatter:
         """``(tensors, cols)`` for the fused scatter, or None when some
         gradient needs the per-name path (unknown name, other shape, dtype or
         device) or the metadata contradicts itself (the views refuse it)."""
+        if type(grads) is not dict:  # any mapping with items()
+            grads = dict(grads.items())
         buf = self._buffer
         dtype, device = buf.dtype, buf.device
         rows = buf.shape[0] if buf.ndim == 2 else math.prod(buf.shape[:-1])

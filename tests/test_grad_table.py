@@ -4,6 +4,9 @@ gradient can have ends up in the same columns (CPU key)."""
 
 from __future__ import annotations
 
+from collections import OrderedDict
+from types import MappingProxyType
+
 import pytest
 import torch
 
@@ -92,6 +95,30 @@ def test_unknown_name_is_refused_and_views_still_alias():
     assert list(view.keys()) == list(SHAPES)
     view["b"].fill_(2.0)
     assert bool((state.grads[:, 6:9] == 2.0).all())
+
+
+class ItemsOnly:
+    """A mapping of which only items() and the length are there."""
+
+    def __init__(self, d):
+        self._d = d
+
+    def __len__(self):
+        return len(self._d)
+
+    def items(self):
+        return self._d.items()
+
+
+@pytest.mark.parametrize("kind", [ItemsOnly, MappingProxyType, OrderedDict])
+@pytest.mark.parametrize("names", ["abcd", "ac"])
+def test_mappings(kind, names):
+    state, other = make(), make()
+    grads = {k: g for k, g in grads_of().items() if k in names}
+    SGD.apply_gradient(state, kind(grads))
+    SGD.apply_gradient(other, grads)
+    assert torch.equal(state.params, other.params)
+    assert torch.equal(state.grads, other.grads) and bool(state.grads.any())
 
 
 @pytest.mark.parametrize("bad", [("a", (4, 3, 2), 0, 5), ("b", (4, 3), 6, 4)])
