@@ -30,6 +30,7 @@ from functools import cached_property
 from typing import Any
 
 import torch
+from torch.autograd import forward_ad
 from torch.func import stack_module_state
 from torch.nn import Module
 
@@ -133,6 +134,8 @@ class _GradScatter:
         buf = self._buffer
         dtype, device = buf.dtype, buf.device
         rows = buf.shape[0] if buf.ndim == 2 else math.prod(buf.shape[:-1])
+        # A dual tensor carries its tangent without requires_grad.
+        tracked = forward_ad._current_level >= 0
         tensors, cols = [], []
         for name, shape, off, n in self._metadata:  # shape: the stacked (N, *shape)
             g = grads.get(name, _ABSENT)
@@ -144,7 +147,7 @@ class _GradScatter:
                     or g.numel() != rows * n
                     or (g.shape != shape and tuple(g.shape) != tuple(shape))):
                 return None
-            tensors.append(g.detach() if g.requires_grad else g)
+            tensors.append(g.detach() if tracked or g.requires_grad else g)
             cols.append(off)
         if len(tensors) != len(grads):  # a name the buffer does not have
             return None

@@ -9,6 +9,7 @@ from types import MappingProxyType
 
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 import churten_amd.kernels  # noqa: F401
 from churten_amd.optimizer import SGD
@@ -119,6 +120,21 @@ def test_mappings(kind, names):
     SGD.apply_gradient(other, grads)
     assert torch.equal(state.params, other.params)
     assert torch.equal(state.grads, other.grads) and bool(state.grads.any())
+
+
+@pytest.mark.parametrize("names", ["abcd", "ac"])
+def test_dual_gradients_leave_no_tangent(names):
+    """The state is plain data: a forward-mode gradient's tangent does not get
+    into its buffers."""
+    state, other = make(), make()
+    grads = {k: g for k, g in grads_of().items() if k in names}
+    with forward_ad.dual_level():
+        SGD.apply_gradient(state, {k: forward_ad.make_dual(g, torch.ones_like(g))
+                                   for k, g in grads.items()})
+        for t in (state.params, state.grads):
+            assert forward_ad.unpack_dual(t).tangent is None
+    SGD.apply_gradient(other, grads)
+    assert torch.equal(state.params, other.params) and torch.equal(state.grads, other.grads)
 
 
 @pytest.mark.parametrize("bad", [("a", (4, 3, 2), 0, 5), ("b", (4, 3), 6, 4)])
