@@ -1390,8 +1390,14 @@ __device__ __forceinline__ T bumped(T x, bool bump) {
 }
 
 // Replica r's step as the scalar cache has it, from before the bump or from
-// after it. It is read once: step_is, before the look into the entry, waits for
-// it and keeps the compiler from reading it again after.
+// after it. The compiler may repeat a load through the constant address space
+// wherever its value is used, and two reads may differ here. The constants come
+// from one value, step_is's: it waits for the load before the look into the
+// entry's memory and nothing after it reads the step again. (The scalar look may
+// be moved: what it finds is right whenever it was read.) loads_state's value is
+// a guess only, which skips_state corrects, so it may be from another read; one
+// value for both (a move through a vector register) cost the smallest SGD calls
+// 1-2%.
 template <typename T>
 __device__ __forceinline__ StepBits<T> step_read(const T* steps, uint32_t r) {
   const uintptr_t at = reinterpret_cast<uintptr_t>(steps + r);
