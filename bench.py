@@ -1145,13 +1145,11 @@ def main():
               "sgd": "SgdPolicy<float, %s, %s, float>" % (
                   "true" if op_args[2] is not None else "false", str(kw.get("nesterov")).lower()),
               "adagrad": "AdagradPolicy<float, float>"}[op_name]
-    # the instantiation the operator launches: ANY = false (State's layout), PRE (per-replica
-    # constants from the workspace: Adam and Adagrad), SMALL (operands of up to 100 MiB,
-    # which the MALL keeps between steps)
+    # the instantiation the operator launches: ANY = false (State's layout), FORM = 2 (a single
+    # launch), SMALL (operands of up to 100 MiB, which the MALL keeps between steps)
     n_rt = sum(t is not None and t.dim() == 2 for t in op_args)
     small = op_args[0].numel() * 4 * n_rt <= 100 << 20
-    kernel = "stream_kernel<%s, false, %s, %s>" % (policy, str(op_name != "sgd").lower(),
-                                                  str(small).lower())
+    kernel = "stream_kernel<%s, false, 2, %s>" % (policy, str(small).lower())
     profile_key = f"{op_name}_stream_kernel_cfg{args.config}"
     hypers = host_hypers(op_name, op_args)
     del op_args

@@ -365,14 +365,18 @@ __device__ __forceinline__ void stream_tile_of_block(const Grid& g, uint32_t& r,
   t0 = int64_t(m - r * g.tiles_per_row + 1) * TILE;
 }
 
-// Replica r's hyperparameter. No kernel writes these vectors, so they are read
-// as constants: with a workgroup's one r that is a scalar load whatever the
-// kernel stores elsewhere. A 16-bit value comes out of the aligned dword that
-// holds it (which never leaves the value's page; there is no 16-bit scalar
-// load).
-template <typename T>
+// Replica r's hyperparameter. CONST (a single launch): read as a constant, which
+// it is, since no kernel writes these vectors. With a workgroup's one r that is a
+// scalar load although the heads store elsewhere; a 16-bit value comes out of the
+// aligned dword that holds it (which never leaves the value's page; there is no
+// 16-bit scalar load). Launches behind a preparation or a bump leave it to the
+// compiler: with constants float64 Adam lost 1-3% and 16-bit Adam up to 6% in
+// segmented launches of 0.8-8 GB, float16 Adagrad 6% in dense ones.
+template <bool CONST, typename T>
 __device__ __forceinline__ double hyper_at(const T* h, uint32_t r) {
-  if constexpr (sizeof(T) == 2) {
+  if constexpr (!CONST) {
+    return static_cast<double>(widen(h[r]));
+  } else if constexpr (sizeof(T) == 2) {
     const uintptr_t at = reinterpret_cast<uintptr_t>(h + r);
     const auto* word =
         reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(at & ~uintptr_t(3));
@@ -666,9 +670,10 @@ struct AdamPolicy {
   // packs to one when the call became a single launch (whole calls, same
   // process: 34 / 51 / 68 / 85 MB of float32 operands +5% / +4% / +2% / +5%, with
   // amsgrad -1% to +6%, float64 -3% to +16%; 128 and 256 threads 4-8% slower, the
-  // scalar read +-1%). With a preparation launch in front (a capture, a smaller
-  // workspace) two packs had been 6% ahead at 34 MB; the shape follows the form
-  // that the operators run.
+  // scalar read +-1%). Behind a preparation launch (a capture, a smaller
+  // workspace) two packs had been 6% ahead at 34 MB in the kernel that served
+  // both forms; with a kernel of its own one pack is level there with one state
+  // resident and 7% ahead with three in turn (float64 +4% and +6%).
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 1, 1);
   static constexpr bool kScalarMaskSmall =
       !kFp32State<T, S> && !std::is_same<T, double>::value;
@@ -712,14 +717,16 @@ struct AdamPolicy {
   };
   static constexpr int kConstants = 2;
   // The step size and sqrt(v)'s divisor of the bumped step (adam_consts).
+  template <bool CONST>
   __device__ static AdamConsts<M> consts(const Vectors<T>& v, uint32_t r, double step) {
     M bc1, bc2s;
-    adam_bias_corrections<M>(hyper_at(v.h[1], r), hyper_at(v.h[2], r), step, bc1, bc2s);
-    return adam_consts<M>(hyper_at(v.h[0], r), bc1, bc2s);
+    adam_bias_corrections<M>(hyper_at<CONST>(v.h[1], r), hyper_at<CONST>(v.h[2], r), step, bc1, bc2s);
+    return adam_consts<M>(hyper_at<CONST>(v.h[0], r), bc1, bc2s);
   }
+  template <bool CONST>
   __device__ static void derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
-    hypers(v, r, rep);
-    rep.c = consts(v, r, step);
+    hypers<CONST>(v, r, rep);
+    rep.c = consts<CONST>(v, r, step);
   }
   __device__ static void constants(const Rep& rep, double* out) {
     out[0] = static_cast<double>(rep.c.step_size);
@@ -736,8 +743,9 @@ struct AdamPolicy {
   // values to the whole wavefront. Each value comes from the same operations
   // on the same operands as in consts(), so the bits are the same, at about
   // half of consts()'s fp64 instructions.
+  template <bool CONST>
   __device__ static void wave_derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
-    hypers(v, r, rep);
+    hypers<CONST>(v, r, rep);
     const bool odd = (__lane_id() & 1) != 0;
     const double bc = adam_bias_correction(odd ? rep.h.beta2 : rep.h.beta1,
                                            static_cast<float>(step));
@@ -754,12 +762,13 @@ struct AdamPolicy {
       rep.c.bc2s_div = wave_lane(x, 1);
     }
   }
+  template <bool CONST>
   __device__ static void hypers(const Vectors<T>& v, uint32_t r, Rep& rep) {
-    rep.h.lr = hyper_at(v.h[0], r);
-    rep.h.beta1 = hyper_at(v.h[1], r);
-    rep.h.beta2 = hyper_at(v.h[2], r);
-    rep.h.eps = hyper_at(v.h[3], r);
-    rep.h.weight_decay = hyper_at(v.h[4], r);
+    rep.h.lr = hyper_at<CONST>(v.h[0], r);
+    rep.h.beta1 = hyper_at<CONST>(v.h[1], r);
+    rep.h.beta2 = hyper_at<CONST>(v.h[2], r);
+    rep.h.eps = hyper_at<CONST>(v.h[3], r);
+    rep.h.weight_decay = hyper_at<CONST>(v.h[4], r);
   }
   __device__ static bool reads_state(const Vectors<T>&, uint32_t) { return true; }
   static constexpr bool kSkipsState = false;
@@ -841,15 +850,17 @@ struct SgdPolicy {
     bool first;
   };
   static constexpr int kConstants = 1;
+  template <bool CONST>
   __device__ static void hypers(const Vectors<T>& v, uint32_t r, Rep& rep) {
-    rep.h.lr = hyper_at(v.h[0], r);
-    rep.h.momentum = hyper_at(v.h[1], r);
-    rep.h.dampening = hyper_at(v.h[2], r);
-    rep.h.weight_decay = hyper_at(v.h[3], r);
+    rep.h.lr = hyper_at<CONST>(v.h[0], r);
+    rep.h.momentum = hyper_at<CONST>(v.h[1], r);
+    rep.h.dampening = hyper_at<CONST>(v.h[2], r);
+    rep.h.weight_decay = hyper_at<CONST>(v.h[3], r);
   }
   // The constant: 1 on the replica's first step, else 0.
+  template <bool CONST>
   __device__ static void derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
-    hypers(v, r, rep);
+    hypers<CONST>(v, r, rep);
     rep.first = step == 1.0;
   }
   __device__ static void constants(const Rep& rep, double* out) { out[0] = rep.first ? 1.0 : 0.0; }
@@ -936,16 +947,18 @@ struct AdagradPolicy {
   };
   static constexpr int kConstants = 1;
   // The constant is corrected_lr of the bumped step.
+  template <bool CONST>
   __device__ static void derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
-    hypers(v, r, rep);
-    rep.h.corrected_lr = adagrad_corrected_lr(hyper_at(v.h[0], r), hyper_at(v.h[1], r),
+    hypers<CONST>(v, r, rep);
+    rep.h.corrected_lr = adagrad_corrected_lr(hyper_at<CONST>(v.h[0], r), hyper_at<CONST>(v.h[1], r),
                                               static_cast<float>(step));
   }
   __device__ static void constants(const Rep& rep, double* out) { out[0] = rep.h.corrected_lr; }
   __device__ static void set(const double* w, Rep& rep) { rep.h.corrected_lr = w[0]; }
+  template <bool CONST>
   __device__ static void hypers(const Vectors<T>& v, uint32_t r, Rep& rep) {
-    rep.h.weight_decay = hyper_at(v.h[2], r);
-    rep.h.eps = hyper_at(v.h[3], r);
+    rep.h.weight_decay = hyper_at<CONST>(v.h[2], r);
+    rep.h.eps = hyper_at<CONST>(v.h[3], r);
     rep.once = kVariant && ilp_row(v.ilp_rows, r);
   }
   __device__ static bool reads_state(const Vectors<T>&, uint32_t) { return true; }
@@ -1053,10 +1066,11 @@ struct AdagradF32Policy {
     AdagradF32Hyper h;
   };
   static constexpr int kConstants = 1;
+  template <bool CONST>
   __device__ static void derive(const Vectors<T>& v, uint32_t r, double step, Rep& rep) {
-    hypers(v, r, rep);
+    hypers<CONST>(v, r, rep);
     rep.h.corrected_lr =
-        adagrad_corrected_lr_f32(hyper_at(v.h[0], r), hyper_at(v.h[1], r), step);
+        adagrad_corrected_lr_f32(hyper_at<CONST>(v.h[0], r), hyper_at<CONST>(v.h[1], r), step);
   }
   __device__ static void constants(const Rep& rep, double* out) {
     out[0] = static_cast<double>(rep.h.corrected_lr);
@@ -1064,11 +1078,12 @@ struct AdagradF32Policy {
   __device__ static void set(const double* w, Rep& rep) {
     rep.h.corrected_lr = static_cast<float>(w[0]);
   }
+  template <bool CONST>
   __device__ static void hypers(const Vectors<T>& v, uint32_t r, Rep& rep) {
-    const double wd = hyper_at(v.h[2], r);
+    const double wd = hyper_at<CONST>(v.h[2], r);
     rep.h.weight_decay = static_cast<float>(wd);
     rep.h.has_weight_decay = wd != 0.0;
-    rep.h.eps = static_cast<float>(hyper_at(v.h[3], r));
+    rep.h.eps = static_cast<float>(hyper_at<CONST>(v.h[3], r));
   }
   __device__ static bool reads_state(const Vectors<T>&, uint32_t) { return true; }
   static constexpr bool kSkipsState = false;
@@ -1087,6 +1102,25 @@ struct AdagradF32Policy {
 template <typename P>
 constexpr int state_slots() {
   return P::NS > 0 ? P::NS : 1;
+}
+
+// How a call comes by its per-replica constants, and by the bumped step: derived
+// in every workgroup behind a bump launch, read from the workspace behind a
+// preparation launch, or in a single launch ("One launch per call"). Each has
+// kernels of its own: a test at run time for the last cost the others (SGD
+// without a workspace 2.3% at 128 x 25.2M parameters, 9.63 -> 9.85 ms, and 1-3%
+// from 0.8 GB of operands on).
+constexpr int kDerived = 0;
+constexpr int kPrepared = 1;
+constexpr int kSingle = 2;
+template <int FORM>
+using Form = std::integral_constant<int, FORM>;
+
+// Whether a form's launch shapes are those of a call with a workspace (PRE
+// below); SGD has one set.
+template <typename P, int FORM>
+constexpr bool pre_of() {
+  return FORM != kDerived && P::kPreWords > 0;
 }
 
 // Packs per thread and residency reservation of the streaming driver, with
@@ -1165,23 +1199,23 @@ template <typename P>
 struct wave_prologue_of<P, std::void_t<decltype(P::kWavePrologue)>> {
   static constexpr bool value = P::kWavePrologue;
 };
-template <typename P>
+template <typename P, bool CONST>
 __device__ __forceinline__ void uniform_derive(const Vectors<typename P::T>& v, uint32_t r,
                                                double step, typename P::Rep& rep) {
   if constexpr (wave_prologue_of<P>::value) {
-    P::wave_derive(v, r, step, rep);
+    P::template wave_derive<CONST>(v, r, step, rep);
   } else {
-    P::derive(v, r, step, rep);
+    P::template derive<CONST>(v, r, step, rep);
   }
 }
 template <typename P, bool PRE>
 __device__ __forceinline__ void prologue(const Vectors<typename P::T>& v, uint32_t r,
                                          typename P::Rep& rep) {
   if constexpr (PRE) {
-    P::hypers(v, r, rep);
+    P::template hypers<false>(v, r, rep);
     P::set(v.pre + kPreStride * r, rep);
   } else {
-    P::derive(v, r, step_at(v.steps, r), rep);
+    P::template derive<false>(v, r, step_at(v.steps, r), rep);
   }
 }
 template <typename P, bool PRE>
@@ -1190,7 +1224,7 @@ __device__ __forceinline__ void uniform_prologue(const Vectors<typename P::T>& v
   if constexpr (PRE) {
     prologue<P, true>(v, r, rep);
   } else {
-    uniform_derive<P>(v, r, step_at(v.steps, r), rep);
+    uniform_derive<P, false>(v, r, step_at(v.steps, r), rep);
   }
 }
 
@@ -1421,14 +1455,17 @@ __device__ __forceinline__ B step_is(B x) {
   }
 }
 
-// Whether the state's loads are issued before the constants are known: in a
-// single-launch call from the step as read, else from the step.
-template <typename P>
+// Whether the state's loads are issued before the constants are known: from the
+// step, or in a single launch from the step as read.
+template <typename P, bool SINGLE>
 __device__ __forceinline__ bool loads_state(const Vectors<typename P::T>& v, uint32_t r,
-                                            bool single, StepBits<typename P::T> x) {
-  if (!single) return P::reads_state(v, r);
-  const auto read = __builtin_bit_cast(typename P::T, x);
-  return P::may_read_state(read, bumped(read, v.one.bump));
+                                            StepBits<typename P::T> x) {
+  if constexpr (!SINGLE) {
+    return P::reads_state(v, r);
+  } else {
+    const auto read = __builtin_bit_cast(typename P::T, x);
+    return P::may_read_state(read, bumped(read, v.one.bump));
+  }
 }
 
 // The constants of a replica every lane of the wavefront works on, in a
@@ -1450,7 +1487,7 @@ __device__ __forceinline__ void single_constants(const Vectors<typename P::T>& v
   const uint64_t word = look ? entry_load<N>(one, r) : 0;
   if (late && entry_is(one, word, w)) return;
   typename P::Rep rep;
-  uniform_derive<P>(v, r, static_cast<double>(widen(step)), rep);
+  uniform_derive<P, true>(v, r, static_cast<double>(widen(step)), rep);
   P::constants(rep, w);
 #pragma unroll
   for (int k = 0; k < N; ++k) {
@@ -1473,18 +1510,15 @@ __device__ __forceinline__ void single_constants(const Vectors<typename P::T>& v
   }
 }
 
-// The same in a call with its preparation (or bump) in a launch before.
-template <typename P, bool PRE>
-__device__ __forceinline__ void call_constants(const Vectors<typename P::T>& v, uint32_t r,
-                                               double (&w)[P::kConstants]) {
-  if constexpr (PRE) {
-#pragma unroll
-    for (int k = 0; k < P::kConstants; ++k) w[k] = v.pre[kPreStride * r + k];
-  } else {
-    typename P::Rep rep;
-    P::derive(v, r, step_at(v.steps, r), rep);
-    P::constants(rep, w);
-  }
+// The replica's constants and hyperparameters in a single launch.
+template <typename P>
+__device__ __forceinline__ void single_prologue(const Vectors<typename P::T>& v, uint32_t r,
+                                                StepBits<typename P::T> x, bool head,
+                                                typename P::Rep& rep) {
+  P::template hypers<true>(v, r, rep);
+  double w[P::kConstants];
+  single_constants<P>(v, r, x, head, w);
+  P::set(w, rep);
 }
 
 // What a head does besides: the zero result, and a frozen replica's step (the
@@ -1678,13 +1712,14 @@ __device__ __forceinline__ void with_maximize(bool maximize, F&& f) {
 // ---------------------------------------------------------------------------
 // Drivers
 // ---------------------------------------------------------------------------
-// PRE: the per-replica constants come from the call's workspace (a.vec.pre).
-// A thread's loads are issued before the replica's prologue, which then runs
-// while they are in flight.
+// FORM: where the per-replica constants come from. A thread's loads are issued
+// before the replica's prologue, which then runs while they are in flight.
 // SMALL: the launch's operands fit the MALL; plain accesses and the small-launch
 // tile instead of non-temporal ones.
-template <typename P, bool ANY, bool PRE, bool SMALL>
+template <typename P, bool ANY, int FORM, bool SMALL>
 __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KArgs<P> a) {
+  constexpr bool PRE = pre_of<P, FORM>();
+  constexpr bool SINGLE = FORM == kSingle;
   constexpr int NTH = stream_threads<P, SMALL>();  // threads per workgroup
   using T = typename P::T;
   using S = typename P::S;
@@ -1702,10 +1737,8 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
   stream_tile_of_block<kStreamTile>(a.g, r, t0);
   const bool active = stream_scalar_mask<P, SMALL>() ? mask_byte_scalar(a.vec.mask, r)
                                                      : a.vec.mask[r] != 0;
-  // In a single-launch call the row's tile 0 is its replica's head.
-  constexpr bool kSingle = PRE || P::kPreWords == 0;
-  const bool single = kSingle && a.vec.one.nonce != 0;
-  const bool is_head = single && t0 == 0 && threadIdx.x < 64;
+  // In a single launch the row's tile 0 is its replica's head.
+  const bool is_head = SINGLE && t0 == 0 && threadIdx.x < 64;
   if (is_head) single_head(a.vec.one, r, active);
   if (!active) return;
 
@@ -1724,8 +1757,8 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
   // the single elements [0, pre) and [body_end, width).
   const auto run = [&](auto head_tile, int64_t first, int64_t packs_left, int64_t pre,
                        int64_t body_end) __attribute__((always_inline)) {
-    const StepBits<T> x = single ? step_read(a.vec.one.steps, r) : StepBits<T>(0);
-    bool load_state = loads_state<P>(a.vec, r, single, x);
+    const StepBits<T> x = SINGLE ? step_read(a.vec.one.steps, r) : StepBits<T>(0);
+    bool load_state = loads_state<P, SINGLE>(a.vec, r, x);
     T* const pbase = pg_row<P>(a.x, 0, r);
     const T* const gbase = pg_row<P>(a.x, 1, r);
     S* sbase[SS];
@@ -1764,17 +1797,12 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
       }
     }
     typename P::Rep rep;
-    if constexpr (kSingle) {
-      P::hypers(a.vec, r, rep);
-      double w[P::kConstants];
-      if (single) {
-        single_constants<P>(a.vec, r, x, is_head, w);
-      } else {
-        call_constants<P, PRE>(a.vec, r, w);
-      }
-      P::set(w, rep);
+    if constexpr (!SINGLE) {
+      uniform_prologue<P, PRE>(a.vec, r, rep);
+    } else {
+      single_prologue<P>(a.vec, r, x, is_head, rep);
       if constexpr (P::kSkipsState) {
-        if (single && !load_state && !P::skips_state(rep)) {
+        if (!load_state && !P::skips_state(rep)) {
           load_state = true;
 #pragma unroll
           for (int u = 0; u < U; ++u) {
@@ -1786,8 +1814,6 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
           }
         }
       }
-    } else {
-      uniform_prologue<P, PRE>(a.vec, r, rep);
     }
     const auto store_packs = [&](int u, int64_t i) {
       store_stream<NT>(prow + i, vp[u]);
@@ -2197,9 +2223,9 @@ __device__ __forceinline__ void seg_singles(const SegTile& t, int64_t numel, Fn&
   }
 }
 
-// Plain accesses in a segmented launch, where the MALL gains by them (CACHE);
-// the rest is non-temporal. Whole calls on three states in turn, same-process
-// A/B:
+// Plain accesses in a segmented single launch, where the MALL gains by them
+// (CACHE); the rest is non-temporal. Whole calls on three states in turn,
+// same-process A/B:
 //   2: every load, for launches whose operands take kSegCacheMin to kMallBytes
 //   (stores of parameters and state stay non-temporal: plain ones +-1%): with
 //   265,484 float32 Adam parameters and the gradient kept, 6 / 8 / 12 / 16 / 20
@@ -2210,13 +2236,19 @@ __device__ __forceinline__ void seg_singles(const SegTile& t, int64_t numel, Fn&
 //   / +7% / +7% / +9%, 32 x 545,100 SGD +6%, but 102 MB -2%, 140 MB and more -3%
 //   to -4%, and under kSegCacheMin -3%.
 // A branch on the launch's kind inside one kernel lost up to 6% of the gain.
+// Behind another launch (captured calls), with the constants first, plain loads
+// gave +5% at 64 MB of operands but -2% to -9% at 34 and -2% to -12% at 90, and
+// the plain gradient store up to -7% at 130: those launches go without.
 constexpr int64_t kSegCacheMin = int64_t(27) << 20;
 constexpr int64_t kSegCacheGrad = int64_t(88) << 20;
 
-// PRE: the per-replica constants come from the call's workspace (a.k.vec.pre).
-// CACHE: plain accesses to the gradient buffer (1) and for every load (2).
-template <typename P, bool ANY, bool PRE, int CACHE = 0>
-__global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(SegArgs<P> a) {
+// FORM: where the per-replica constants come from. CACHE: plain accesses to the
+// gradient buffer (1) and for every load (2).
+template <typename P, bool ANY, int FORM, int CACHE = 0>
+__global__ __launch_bounds__((segment_threads<P, pre_of<P, FORM>()>())) void segment_kernel(
+    SegArgs<P> a) {
+  constexpr bool PRE = pre_of<P, FORM>();
+  constexpr bool SINGLE = FORM == kSingle;
   constexpr bool NTG = CACHE == 0, NTL = CACHE < 2;
   using T = typename P::T;
   using S = typename P::S;
@@ -2232,23 +2264,23 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
   // config 5's per-parameter gradients).
   constexpr int KP = stream_pack<T, S>();
   const uint32_t tiles_per_row = a.seg.tile0[a.seg.n];
-  // A single-launch call's first workgroups are the replicas' heads, which only
-  // make the constants known.
-  constexpr bool kSingle = PRE || P::kPreWords == 0;
-  const bool single = kSingle && a.k.vec.one.nonce != 0;
-  if (blockIdx.x < a.k.g.heads) {
-    const uint32_t r = blockIdx.x;
-    const bool active = mask_byte_scalar(a.k.vec.mask, r);
-    if (threadIdx.x < 64) {
-      single_head(a.k.vec.one, r, active);
-      if (active) {
-        double w[P::kConstants];
-        single_constants<P>(a.k.vec, r, step_read(a.k.vec.one.steps, r), true, w);
+  // A single launch's first workgroups are the replicas' heads, which only make
+  // the constants known.
+  if constexpr (SINGLE) {
+    if (blockIdx.x < a.k.g.heads) {
+      const uint32_t r = blockIdx.x;
+      const bool active = mask_byte_scalar(a.k.vec.mask, r);
+      if (threadIdx.x < 64) {
+        single_head(a.k.vec.one, r, active);
+        if (active) {
+          double w[P::kConstants];
+          single_constants<P>(a.k.vec, r, step_read(a.k.vec.one.steps, r), true, w);
+        }
       }
+      return;
     }
-    return;
   }
-  const uint32_t block = blockIdx.x - a.k.g.heads;
+  const uint32_t block = SINGLE ? blockIdx.x - a.k.g.heads : blockIdx.x;
   const uint32_t r = block / tiles_per_row;
   const uint32_t local = block - r * tiles_per_row;
   const bool write_grad = a.k.x.data[1] != nullptr;
@@ -2301,23 +2333,12 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
     return;
   }
 
+  // Behind another launch the constants are read before the tile's loads are
+  // issued, in a single launch after: the wait for the entry is then hidden.
   typename P::Rep rep;
-  const StepBits<T> x = single ? step_read(a.k.vec.one.steps, r) : StepBits<T>(0);
-  bool load_state = loads_state<P>(a.k.vec, r, single, x);
-  const auto constants = [&]() __attribute__((always_inline)) {
-    if constexpr (kSingle) {
-      P::hypers(a.k.vec, r, rep);
-      double w[P::kConstants];
-      if (single) {
-        single_constants<P>(a.k.vec, r, x, false, w);
-      } else {
-        call_constants<P, PRE>(a.k.vec, r, w);
-      }
-      P::set(w, rep);
-    } else {
-      prologue<P, PRE>(a.k.vec, r, rep);
-    }
-  };
+  if constexpr (!SINGLE) prologue<P, PRE>(a.k.vec, r, rep);
+  const StepBits<T> x = SINGLE ? step_read(a.k.vec.one.steps, r) : StepBits<T>(0);
+  bool load_state = loads_state<P, SINGLE>(a.k.vec, r, x);
   const T zero = narrow<T>(op_t<T>(0));
 
   T* const prow = pg_row<P>(a.k.x, 0, r) + col * a.k.x.stride_t[0];
@@ -2346,8 +2367,10 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
   };
 
   if (!vec) {
-    constants();
-    if constexpr (P::kSkipsState) load_state = load_state || !P::skips_state(rep);
+    if constexpr (SINGLE) {
+      single_prologue<P>(a.k.vec, r, x, false, rep);
+      if constexpr (P::kSkipsState) load_state = load_state || !P::skips_state(rep);
+    }
     const int64_t cnt = imin(kSegTile, numel - j0);
     for (int64_t j = j0 + threadIdx.x; j < j0 + cnt; j += NTH) one(j);
     return;
@@ -2386,17 +2409,19 @@ __global__ __launch_bounds__((segment_threads<P, PRE>())) void segment_kernel(Se
       }
     }
   }
-  constants();
-  if constexpr (P::kSkipsState) {
-    if (single && !load_state && !P::skips_state(rep)) {
-      load_state = true;
+  if constexpr (SINGLE) {
+    single_prologue<P>(a.k.vec, r, x, false, rep);
+    if constexpr (P::kSkipsState) {
+      if (!load_state && !P::skips_state(rep)) {
+        load_state = true;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t i = int64_t(u) * NTH + threadIdx.x;
-        if (i < t.packs) {
+        for (int u = 0; u < U; ++u) {
+          const int64_t i = int64_t(u) * NTH + threadIdx.x;
+          if (i < t.packs) {
 #pragma unroll
-          for (int b = 0; b < NS; ++b) {
-            vs[b][u] = Packs<ANY, S, NTL, KP>(srow[b] + t.first).load(i);
+            for (int b = 0; b < NS; ++b) {
+              vs[b][u] = Packs<ANY, S, NTL, KP>(srow[b] + t.first).load(i);
+            }
           }
         }
       }
@@ -2530,7 +2555,8 @@ __global__ __launch_bounds__(kThreads) void prep_kernel(Vectors<typename P::T> v
     }
     if (active) {
       typename P::Rep rep;
-      P::derive(v, static_cast<uint32_t>(r), step_at(v.steps, static_cast<uint32_t>(r)), rep);
+      P::template derive<false>(v, static_cast<uint32_t>(r),
+                                step_at(v.steps, static_cast<uint32_t>(r)), rep);
       P::constants(rep, pre + kPreStride * r);
     }
   }
@@ -2967,18 +2993,20 @@ void launch_column(const ColArgs<P>& ca, uint32_t blocks, bool private_lines,
 
 // The streaming driver over `blocks` tiles, capped when the launch is large
 // (`mid`: the operands take at most kMidBytes; with a workspace only).
-template <typename P, bool PRE, bool SMALL>
-void launch_stream(const KArgs<P>& a, uint32_t blocks, bool same_phase, hipStream_t stream,
-                   bool mid = false) {
+template <typename P, int FORM, bool SMALL>
+int launch_stream(const KArgs<P>& a, uint32_t blocks, bool same_phase, hipStream_t stream,
+                  bool mid) {
+  constexpr bool PRE = pre_of<P, FORM>();
   const uint32_t cap = PRE && !SMALL && mid ? P::kStreamLdsMid : stream_lds_of<P, PRE, SMALL>();
   const uint32_t lds = int64_t(blocks) * stream_tile<P, PRE, SMALL>() >= kCapMinElems ? cap : 0u;
   if (same_phase) {
-    hipLaunchKernelGGL((stream_kernel<P, false, PRE, SMALL>), dim3(blocks),
+    hipLaunchKernelGGL((stream_kernel<P, false, FORM, SMALL>), dim3(blocks),
                        dim3(stream_threads<P, SMALL>()), lds, stream, a);
   } else {
-    hipLaunchKernelGGL((stream_kernel<P, true, PRE, SMALL>), dim3(blocks),
+    hipLaunchKernelGGL((stream_kernel<P, true, FORM, SMALL>), dim3(blocks),
                        dim3(stream_threads<P, SMALL>()), lds, stream, a);
   }
+  return static_cast<int>(hipGetLastError());
 }
 
 // Consolidated-gradient update with policy P over `nbufs` operands.
@@ -2989,8 +3017,6 @@ int launch_dense(const Call& c, int nbufs) {
   bool streamable = false;
   const bool pre = uses_workspace<P>(c);
   // Operands that fit the MALL (R, T and the types say so, before any launch).
-  // The small shape is built for the forms the operators run: with a
-  // workspace where the policy has one, and for SGD, which has none.
   const bool small =
       (pre || P::kPreWords == 0) &&
       c.R <= kMallBytes / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1) &&
@@ -3023,23 +3049,22 @@ int launch_dense(const Call& c, int nbufs) {
     uint32_t col_blocks = 0;
     if (streamable) {
       const bool same_phase = rows_same_phase<P>(a.x, nbufs, P::kStreamPack);
-      if constexpr (P::kPreWords > 0) {
-        if (pre) {
-          if (small) {
-            launch_stream<P, true, true>(a, blocks, same_phase, c.stream);
-          } else {
-            launch_stream<P, true, false>(a, blocks, same_phase, c.stream, mid);
-          }
-          return static_cast<int>(hipGetLastError());
-        }
+      const auto launch = [&](auto form, auto is_small) {
+        return launch_stream<P, decltype(form)::value, decltype(is_small)::value>(
+            a, blocks, same_phase, c.stream, mid);
+      };
+      // The small shape is built for the forms the operators run: with a
+      // workspace where the policy has one, and for SGD, which has none.
+      if (a.vec.one.nonce != 0) {
+        return small ? launch(Form<kSingle>(), std::true_type{})
+                     : launch(Form<kSingle>(), std::false_type{});
       }
-      if constexpr (P::kPreWords == 0) {
-        if (small) {
-          launch_stream<P, false, true>(a, blocks, same_phase, c.stream);
-          return static_cast<int>(hipGetLastError());
-        }
+      constexpr int kBehind = P::kPreWords > 0 ? kPrepared : kDerived;
+      if (pre || P::kPreWords == 0) {
+        return small ? launch(Form<kBehind>(), std::true_type{})
+                     : launch(Form<kBehind>(), std::false_type{});
       }
-      launch_stream<P, false, false>(a, blocks, same_phase, c.stream);
+      return launch(Form<kDerived>(), std::false_type{});
     } else if (replica_minor(a.x, nbufs) && make_col_grid(c.R, c.T, ca.g, col_blocks)) {
       ca.x = a.x;
       ca.vec = a.vec;
@@ -3112,30 +3137,31 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
       return launch_walk<T>(walk, c.R, tile, vec_rows, a, a.seg, kernel, c.stream, lds, nth,
                             heads);
     };
-    // The forms the operators run (with a workspace where the policy has one)
-    // come with plain accesses too, for operands that share a phase.
-    constexpr bool kCached = P::kPreWords == 0;
-    if constexpr (P::kPreWords > 0) {
-      if (pre) {
-        constexpr int nth = segment_threads<P, true>();
-        // the cap only where it can pay (as for the streaming driver's
-        // launches: at least kCapMinElems elements)
-        const uint32_t lds = c.R * c.T >= kCapMinElems
-                                 ? segment_lds<P>(large, a.k.x.data[1] != nullptr)
-                                 : 0u;
-        if (!same_phase) return launch(segment_kernel<P, true, true>, lds, nth);
-        if (cache == 2) return launch(segment_kernel<P, false, true, 2>, lds, nth);
-        if (cache == 1) return launch(segment_kernel<P, false, true, 1>, lds, nth);
-        return launch(segment_kernel<P, false, true>, lds, nth);
+    // The cap only where it can pay (as for the streaming driver's launches: at
+    // least kCapMinElems elements).
+    const bool capped = c.R * c.T >= kCapMinElems;
+    if (a.k.vec.one.nonce != 0) {
+      constexpr int nth = segment_threads<P, pre_of<P, kSingle>()>();
+      uint32_t lds = 0;
+      if constexpr (pre_of<P, kSingle>()) {
+        if (capped) lds = segment_lds<P>(large, a.k.x.data[1] != nullptr);
       }
+      if (!same_phase) return launch(segment_kernel<P, true, kSingle>, lds, nth);
+      if (cache == 2) return launch(segment_kernel<P, false, kSingle, 2>, lds, nth);
+      if (cache == 1) return launch(segment_kernel<P, false, kSingle, 1>, lds, nth);
+      return launch(segment_kernel<P, false, kSingle>, lds, nth);
     }
-    constexpr int nth = segment_threads<P, false>();
-    if (!same_phase) return launch(segment_kernel<P, true, false>, 0, nth);
-    if constexpr (kCached) {
-      if (cache == 2) return launch(segment_kernel<P, false, false, 2>, 0, nth);
-      if (cache == 1) return launch(segment_kernel<P, false, false, 1>, 0, nth);
+    const auto behind = [&](auto form) {
+      constexpr int F = decltype(form)::value;
+      constexpr int nth = segment_threads<P, pre_of<P, F>()>();
+      const uint32_t lds = pre_of<P, F>() && capped ? segment_lds_pre_of<P>::value : 0u;
+      return same_phase ? launch(segment_kernel<P, false, F>, lds, nth)
+                        : launch(segment_kernel<P, true, F>, lds, nth);
+    };
+    if constexpr (P::kPreWords > 0) {
+      if (pre) return behind(Form<kPrepared>());
     }
-    return launch(segment_kernel<P, false, false>, 0, nth);
+    return behind(Form<kDerived>());
   });
 }
 
