@@ -463,6 +463,25 @@ constexpr int64_t small_from(int64_t wide, int64_t narrow) {
   return (sizeof(T) == 2 ? narrow : wide) << 20;
 }
 
+// From this many bytes of operands a policy's calls that could run as a single
+// launch (kBehindDense, segmented with the gradients kept kBehindKept, not kept
+// kBehindFused) take two: beyond it the look into the entry costs every tile more
+// than the second launch costs the call. Whole calls, single / two launches, same
+// process, mean over 8 and 24 rows; the policies that are not named here stay
+// level or gain as a single launch.
+//   float32 Adam fused 1.2 / 2 / 4 / 8 GB 0.992 / 0.956 / 0.978 / 0.958 (0.5-0.8
+//     GB 1.006-1.002), with bfloat16 moments 2 / 4 / 8 GB 0.993 / 0.974 / 0.992;
+//   float64 Adam fused 0.8 / 2 / 4 GB 0.986 / 0.974 / 0.962 (0.5 GB 1.004);
+//   16-bit Adam kept 2 / 4 / 8 GB 0.986 / 0.960 / 0.952 bfloat16, 1.004 / 0.988 /
+//     0.973 float16, with amsgrad 0.6 / 0.8 / 1.2 / 2 GB 0.983 / 0.977 / 0.957 /
+//     0.948; bfloat16 fused 2 / 4 GB 0.986 / 0.985;
+//   Adagrad with bfloat16 state dense 0.8 / 2 / 8 GB 0.991 / 0.982 / 0.987, fused 2
+//     / 4 / 8 GB 0.987 / 0.980 / 0.969, bfloat16 kept 4 / 8 GB 0.984 / 0.968;
+//   in float32 math, bfloat16 state, fused 0.8 / 2 / 4 GB 0.991 / 0.970 / 0.966,
+//     bfloat16 params fused 2 / 4 GB 0.982 / 0.984.
+constexpr int64_t kNever = INT64_MAX;
+constexpr int64_t kMiB = int64_t(1) << 20;
+
 // Launches above the MALL with at most kMidBytes of (R, T) operands reserve
 // each policy's kStreamLdsMid instead of its large-launch cap (with a
 // workspace). Measured with a launch-shape sweep at config 2's size (100 x 265,484,
@@ -710,6 +729,13 @@ struct AdamPolicy {
   static constexpr uint32_t kSegmentLdsFused = kFp32State<T, S> ? lds_for_residency(14) : 0u;
   static constexpr bool kLateStores = !AMSGRAD && std::is_same<T_, float>::value;
   static constexpr bool kVariant = false;
+  static constexpr int64_t kBehindDense = kNever;
+  static constexpr int64_t kBehindKept = sizeof(T) != 2 ? kNever : (AMSGRAD ? 560 : 1536) * kMiB;
+  static constexpr int64_t kBehindFused =
+      std::is_same<T, double>::value                        ? 640 * kMiB
+      : kFp32State<T, S>                                    ? (AMSGRAD ? kNever : 1024 * kMiB)
+      : kBf16State<T, S> || std::is_same<T, bf16_t>::value ? 1536 * kMiB
+                                                            : kNever;
   static constexpr int kPreWords = 2;
   struct Rep {
     AdamHyper h;
@@ -844,6 +870,9 @@ struct SgdPolicy {
   static constexpr bool kSegmentScalarMask = true;
   static constexpr bool kLateStores = std::is_same<T_, float>::value;
   static constexpr bool kVariant = false;
+  static constexpr int64_t kBehindDense = kNever;
+  static constexpr int64_t kBehindKept = kNever;
+  static constexpr int64_t kBehindFused = kNever;
   static constexpr int kPreWords = 0;
   struct Rep {
     SgdHyper<double> h;
@@ -940,6 +969,10 @@ struct AdagradPolicy {
   static constexpr bool kSegmentScalarMask = true;
   static constexpr bool kLateStores = false;
   static constexpr bool kVariant = std::is_same_v<T, _Float16> && std::is_same_v<S, _Float16>;
+  static constexpr int64_t kBehindDense = kBf16State<T, S> ? 640 * kMiB : kNever;
+  static constexpr int64_t kBehindKept =
+      std::is_same<T, bf16_t>::value ? 3072 * kMiB : kNever;
+  static constexpr int64_t kBehindFused = kBf16State<T, S> ? 1536 * kMiB : kNever;
   static constexpr int kPreWords = 1;
   struct Rep {
     AdagradHyper h;
@@ -1061,6 +1094,11 @@ struct AdagradF32Policy {
   static constexpr bool kSegmentScalarMask = true;
   static constexpr bool kLateStores = false;
   static constexpr bool kVariant = false;
+  static constexpr int64_t kBehindDense = kNever;
+  static constexpr int64_t kBehindKept = kNever;
+  static constexpr int64_t kBehindFused = kBf16State<T, S>                  ? 640 * kMiB
+                                          : std::is_same<T, bf16_t>::value ? 1536 * kMiB
+                                                                            : kNever;
   static constexpr int kPreWords = 1;
   struct Rep {
     AdagradF32Hyper h;
@@ -3052,7 +3090,8 @@ int launch_dense(const Call& c, int nbufs) {
     if (!make_grid(c.R, c.T, tile, a.g, blocks, threads, streamable)) return false;
     a.g.res0 = res0;
     a.g.rmod = rmod;
-    if (streamable && single_launch(c)) {
+    if (streamable && c.R * c.T * operand_bytes_per_elem<P>() < P::kBehindDense &&
+        single_launch(c)) {
       a.vec.one = single_of<typename P::T>(c, kEarlyBlocks);
     }
     return true;
@@ -3139,7 +3178,10 @@ int launch_segments(const Call& c, int nbufs, const ts_segment* segs, int n_segs
     // No more workgroups than this, heads included: T / tile, the last tile of
     // every segment and of every gap, and one head, per replica.
     const uint64_t most = static_cast<uint64_t>(c.R) * (c.T / tile + 2 * n_segs + 3);
-    if (grid_fits(most, nth) && single_launch(c)) a.k.vec.one = single_of<T>(c, 0);
+    if (grid_fits(most, nth) && bytes < (keeps ? P::kBehindKept : P::kBehindFused) &&
+        single_launch(c)) {
+      a.k.vec.one = single_of<T>(c, 0);
+    }
     return true;
   };
   return run_step<P>(c, a.k.vec, prepare, [&]() -> int {

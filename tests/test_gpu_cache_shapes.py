@@ -96,6 +96,11 @@ def test_dense_sizes(opt, dtype, state, nbytes):
     check(opt, dtype, state, nbytes, segmented=False)
 
 
+@pytest.mark.parametrize("nbytes", [639 * MB, 641 * MB])
+def test_dense_sizes_in_one_and_two_launches(nbytes):
+    check("adagrad", torch.float32, torch.bfloat16, nbytes, segmented=False)
+
+
 @pytest.mark.parametrize("nbytes", [26 * MB, 28 * MB, 99 * MB, 101 * MB, 430 * MB, 450 * MB])
 @pytest.mark.parametrize("opt,dtype,state", [
     ("adam", torch.float32, torch.float32), ("adam", torch.float32, torch.bfloat16),
