@@ -444,10 +444,13 @@ constexpr int64_t kCapMinElems = int64_t(8192) * 512;
 // (so three times the operands pass between two steps of one), plain against
 // non-temporal, same process: float32 Adam at 34 / 51 / 85 / 102 / 119 / 136 /
 // 238 MB 11.9 / 16.1 / 25.3 / 31.1 / 39.9 / 47.9 / 80.3 us against 12.9 / 17.4 /
-// 26.5 / 30.4 / 34.7 / 39.2 / 65.9, and every other optimizer and type crosses
-// between 84 and 131 MB too (16-bit Adagrad at 130-200). With one state alone,
-// plain accesses win up to 209 MB (config 3 32.0 us against 35.8), but then
-// nothing else may pass through the cache between steps.
+// 26.5 / 30.4 / 34.7 / 39.2 / 65.9, and every other optimizer and type but float16
+// Adagrad crosses between 84 and 131 MB too. With one state alone, and nothing
+// else through the cache between its steps, plain accesses stay ahead to the
+// MALL's size: by 0-4% from 130 to 240 MB in float32 Adam and SGD, 4-9% in 16-bit
+// Adam (bfloat16 Adagrad 5-10%; 16-bit SGD loses there too), against the 10-30%
+// that they lose on three states. A training step's activations and gradients
+// pass through the cache, so the line follows the second.
 constexpr int64_t kMallBytes = int64_t(100) << 20;
 
 // The smallest launches of some policies take the large shape too
@@ -696,6 +699,7 @@ struct AdamPolicy {
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 1, 1);
   static constexpr bool kScalarMaskSmall =
       !kFp32State<T, S> && !std::is_same<T, double>::value;
+  static constexpr int64_t kStreamSmallTo = kMallBytes;
   static constexpr int64_t kStreamSmallFrom =
       std::is_same<T, bf16_t>::value ? int64_t(48) << 20 : int64_t(28) << 20;
   static constexpr int kStreamPack = stream_pack<T, S>();
@@ -852,6 +856,7 @@ struct SgdPolicy {
   // and 6.88-6.93 for 256; with the scalar read 256 threads ran 2.2% ahead of
   // 128 (same-process A/B, 10 rounds).
   static constexpr int kStreamBlockSmall = kFp32State<T, S> ? 256 : kStreamThreads;
+  static constexpr int64_t kStreamSmallTo = kMallBytes;
   static constexpr int64_t kStreamSmallFrom =
       small_from<T>(std::is_same<T, double>::value ? 16 : 0, 48);
   static constexpr int kStreamPack = stream_pack<T, S>();
@@ -950,6 +955,12 @@ struct AdagradPolicy {
   // 19-97 MB).
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 1, 1);
   static constexpr bool kScalarMaskSmall = sizeof(T) == 2;
+  // float16 keeps plain accesses up to the MALL's size: from 110 to 240 MB they
+  // are 15-20% ahead with one state resident (110 / 160 / 240 MB 33.3 / 46.1 /
+  // 68.0 us against 40.2 / 55.1 / 79.2) and 4-10% with three in turn (38.7 / 54.9
+  // / 78.7 against 42.7 / 57.9 / 82.3).
+  static constexpr int64_t kStreamSmallTo =
+      std::is_same<T, _Float16>::value ? int64_t(256) << 20 : kMallBytes;
   static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
   static constexpr int kStreamPack = stream_pack<T, S>();
   // Segmented float32 updates with a workspace: one-wavefront workgroups, one
@@ -1082,6 +1093,7 @@ struct AdagradF32Policy {
   static constexpr bool kScalarMask = std::is_same<T, float>::value;
   // float32: one pack in a single launch (two: -1% to -17% at 19-97 MB).
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 4, 1);
+  static constexpr int64_t kStreamSmallTo = kMallBytes;
   static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
   static constexpr int kStreamPack = stream_pack<T, S>();
   // Segmented with a workspace: one-wavefront workgroups, one pack, the
@@ -3071,7 +3083,7 @@ int launch_dense(const Call& c, int nbufs) {
   // Operands that fit the MALL (R, T and the types say so, before any launch).
   const bool small =
       (pre || P::kPreWords == 0) &&
-      c.R <= kMallBytes / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1) &&
+      c.R <= P::kStreamSmallTo / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1) &&
       c.R * c.T * operand_bytes_per_elem<P>() >= P::kStreamSmallFrom;
   const bool mid =
       c.R <= kMidBytes / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1);
