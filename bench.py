@@ -246,15 +246,19 @@ def abi_update_call(op_name, args, kw, extra_flags: int = 0, dtype_code: int = 0
                     workspace: bool = True):
     """A no-argument function that enqueues one update through the C ABI on
     torch's current stream, without the step bump, and returns its status.
-    Adam and Adagrad go through the workspace entry points, as the operator
-    does (their preparation launch then precedes the update); workspace=False
-    calls the entry points without one."""
+    It goes through the workspace entry points with the operators' workspace, so
+    it is the launch (or, for more than 1024 replicas and for the large calls of
+    some types, the two) that they make; workspace=False calls the entry points
+    without one."""
     import ctypes
 
     import torch
 
     lib = ctypes.CDLL(str(ROOT / "churten_amd" / "lib" / "libchurten_optim.so"))
-    ws = torch.empty(16 * args[0].shape[0], dtype=torch.uint8, device=args[0].device)
+    lib.ts_single_launch_bytes.restype = ctypes.c_size_t
+    replicas = args[0].shape[0]
+    ws_bytes = lib.ts_single_launch_bytes(ctypes.c_int64(replicas)) or 16 * replicas
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=args[0].device)
     ws_args = (ctypes.c_void_p(ws.data_ptr()), ctypes.c_size_t(ws.numel()))
 
     class RtBuf(ctypes.Structure):
@@ -282,10 +286,13 @@ def abi_update_call(op_name, args, kw, extra_flags: int = 0, dtype_code: int = 0
     elif op_name == "sgd":
         bufs = (RtBuf * 3)(*[buf(t) for t in args[:3]])
         flags = (8 if kw["nesterov"] else 0) | extra_flags
-        call = lambda: lib.ts_sgd_step(  # noqa: E731
-            bufs, dtype_code, vp(args[3]), *[vp(t) for t in args[4:8]], vp(args[8]),
-            ctypes.c_int64(R), ctypes.c_int64(T), ctypes.c_uint32(flags),
-            ctypes.c_void_p(0), ctypes.c_void_p(stream.cuda_stream))
+        head = (bufs, dtype_code, vp(args[3]), *[vp(t) for t in args[4:8]], vp(args[8]),
+                ctypes.c_int64(R), ctypes.c_int64(T), ctypes.c_uint32(flags), ctypes.c_void_p(0))
+        if workspace:
+            call = lambda: lib.ts_sgd_step_ws(  # noqa: E731
+                *head, *ws_args, ctypes.c_void_p(stream.cuda_stream))
+        else:
+            call = lambda: lib.ts_sgd_step(*head, ctypes.c_void_p(stream.cuda_stream))  # noqa: E731
     elif op_name == "adagrad":
         bufs = (RtBuf * 3)(*[buf(t) for t in args[:3]])
         head = (bufs, dtype_code, vp(args[3]), *[vp(t) for t in args[4:8]], vp(args[8]),
@@ -308,9 +315,9 @@ def abi_update_call(op_name, args, kw, extra_flags: int = 0, dtype_code: int = 0
 def kernel_only_timing(op_name, args, kw, launches: int, extra_flags: int = 0,
                        dtype_code: int = 0, workspace: bool = True) -> float:
     """Average duration (ms) of the update: `abi_update_call` bracketed by HIP
-    events on the launch stream. With a workspace the preparation launch (the
-    per-replica constants, one tiny kernel) is inside the bracket, a few
-    microseconds against the update's milliseconds at config 5."""
+    events on the launch stream. Where the call takes two launches the
+    preparation (the per-replica constants, one tiny kernel) is inside the
+    bracket, a few microseconds against milliseconds."""
     import torch
 
     call = abi_update_call(op_name, args, kw, extra_flags, dtype_code, workspace)
@@ -331,7 +338,7 @@ EVICT_BYTES = 1 << 30
 
 def mall_residency_timing(op_name, args, kw, nbytes: int, launches: int):
     """Where an update's operands are served from when its launches run back
-    to back: each launch (preparation + update, through the C ABI) timed
+    to back: each call (the operator's launch, through the C ABI) timed
     alone between two HIP events, once with the previous launch right before
     it (operands warm in the 256 MB MALL if they fit) and once with a 1 GiB
     read of another buffer between launches, outside the timed interval,

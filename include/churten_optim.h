@@ -187,10 +187,11 @@ int ts_adagrad_step_segments(const ts_rt_buf* bufs, const ts_segment* grads, int
  *                    invalid argument.
  * Two launches per call (preparation, update), as without a workspace. With a
  * workspace of 128 R bytes or more, R <= 1024, unit inner strides and no
- * capture under way on the stream, the call is one launch: the update bumps the
- * steps and passes the constants on itself, with the same results (the
- * preparation launch costs 2-3.5 us of GPU time). It then also reads what the
- * workspace held before, to tell that it is not its own.
+ * capture under way on the stream, the call is one launch (but for the largest
+ * calls of some types): the update bumps the steps and passes the constants on
+ * itself, with the same results (the preparation launch costs 2-3.5 us of GPU
+ * time). It then also reads what the workspace held before, to tell that it is
+ * not its own.
  * These replace the same reference interfaces as ts_adam_step, ts_adagrad_step
  * and their segmented forms (stubs.cpp:25-41, 61-72; cuda/adam.cu:99-122 and
  * cuda/adagrad.cu:141-148 are the per-block prologues whose constants the
