@@ -429,14 +429,31 @@ def geometry_timing(rows: int, launches: int, rounds: int = 3):
     return out
 
 
+# Operand bytes from which a float32 dense launch takes the small shape; below
+# it the policy runs the large launches' (kStreamSmallFrom in optim_drivers.h).
+SMALL_FROM = {"adam": 28 << 20, "sgd": 0, "adagrad": 16 << 20}
+LAUNCH_CLASSES = ("smallest", "small", "mid", "large")
+
+
+def launch_class(op_name: str, operand_bytes: int) -> str:
+    """The launch shape of a float32 dense update over this many bytes of
+    operands: plain accesses and the small shape from SMALL_FROM to 100 MiB, the
+    large shape under a cap of its own up to 1 GiB ("mid") and above, and
+    uncapped below the small one."""
+    if operand_bytes > 1 << 30:
+        return "large"
+    if operand_bytes > 100 << 20:
+        return "mid"
+    return "small" if operand_bytes >= SMALL_FROM[op_name] else "smallest"
+
+
 def size_sweep_timing(cfg: int, ns, launches: int):
     """The config's update on the first n rows of one allocation of max(ns)
     rows (same buffers, same per-replica hyperparameters and mask, so only
-    the size changes), kernel-only time per launch, and per launch-size class
-    (operands up to 100 MiB: small, up to 1 GiB: mid, above: large; each class
-    has its own launch shape) a least-squares fit t = t0 + bytes / rate: t0 is
-    what a launch costs beyond streaming its bytes (the preparation launch,
-    the grid's ramp-up, the drain of its last workgroups), `rate` the
+    the size changes), kernel-only time per launch, and per launch class
+    (`launch_class`; each has its own shape) a least-squares fit t = t0 + bytes /
+    rate: t0 is what a launch costs beyond streaming its bytes (the launch
+    itself, the grid's ramp-up, the drain of its last workgroups), `rate` the
     streaming rate of that shape."""
     import torch
 
@@ -452,13 +469,13 @@ def size_sweep_timing(cfg: int, ns, launches: int):
         ms = kernel_only_timing(op_name, args, kw, launches)
         opb = n * T * 4 * n_rt
         pts.append({"N": n, "active": active, "bytes": nbytes, "operand_bytes": opb,
-                    "class": "small" if opb <= 100 << 20 else "mid" if opb <= 1 << 30 else "large",
+                    "class": launch_class(op_name, opb),
                     "kernel_avg_us": round(ms * 1e3, 2),
                     "GBs": round(nbytes / (ms * 1e-3) / 1e9, 1)})
     del full, args
     torch.cuda.empty_cache()
     fits = {}
-    for cls in ("small", "mid", "large"):
+    for cls in LAUNCH_CLASSES:
         sel = [p for p in pts if p["class"] == cls]
         if len(sel) >= 3:
             fits[cls] = fit_fixed_and_rate([p["bytes"] for p in sel],
@@ -1153,9 +1170,9 @@ def main():
                   "true" if op_args[2] is not None else "false", str(kw.get("nesterov")).lower()),
               "adagrad": "AdagradPolicy<float, float>"}[op_name]
     # the instantiation the operator launches: ANY = false (State's layout), FORM = 2 (a single
-    # launch), SMALL (operands of up to 100 MiB, which the MALL keeps between steps)
+    # launch), SMALL (operands that the MALL keeps between steps)
     n_rt = sum(t is not None and t.dim() == 2 for t in op_args)
-    small = op_args[0].numel() * 4 * n_rt <= 100 << 20
+    small = launch_class(op_name, op_args[0].numel() * 4 * n_rt) == "small"
     kernel = "stream_kernel<%s, false, 2, %s>" % (policy, str(small).lower())
     profile_key = f"{op_name}_stream_kernel_cfg{args.config}"
     hypers = host_hypers(op_name, op_args)

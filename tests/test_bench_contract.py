@@ -57,3 +57,15 @@ def test_fit_fixed_and_rate_recovers_a_line():
     assert fit["t0_us"] == pytest.approx(4.0, abs=0.01)
     assert fit["rate_GBs"] == pytest.approx(6500.0, rel=1e-4)
     assert fit["max_residual_us"] == pytest.approx(0.0, abs=0.01)
+
+
+@pytest.mark.parametrize("op,edge", [("adam", 28), ("adagrad", 16)])
+def test_launch_classes(op, edge):
+    """The sweep's classes are the dense driver's launch shapes, the one below
+    the small shape included (2 and 4 of config 1's replicas run there)."""
+    mb = 1 << 20
+    sizes = [edge * mb - 1, edge * mb, 100 * mb, 100 * mb + 1, 1024 * mb, 1024 * mb + 1]
+    assert [bench.launch_class(op, n) for n in sizes] == [
+        "smallest", "small", "small", "mid", "mid", "large"]
+    assert bench.launch_class("sgd", 1) == "small"
+    assert bench.launch_class("adam", 4 * 265484 * 16) == "smallest"
