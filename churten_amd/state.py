@@ -26,7 +26,6 @@ from __future__ import annotations
 
 import math
 from collections.abc import Sequence
-from functools import cached_property
 from typing import Any
 
 import torch
@@ -99,25 +98,31 @@ def consolidated_dict_view(tcons: torch.Tensor, metadata) -> dict[str, torch.Ten
     return {name: tcons[..., off : off + n].view(*shape) for name, shape, off, n in metadata}
 
 
-_ABSENT = object()
-
-
 class _GradScatter:
     """The gradient buffer seen through per-name views; ``update_`` writes a
     per-name gradient dict into the consolidated ``(N, T)`` buffer -- in one
     ``churten::scatter_grads_`` launch when every gradient is exactly
     ``(N, *shape)`` in the buffer's dtype and device, else one ``copy_`` per
-    name (which also broadcasts and converts, as the views' ``copy_`` would)."""
+    name (which also broadcasts and converts, as the views' ``copy_`` would).
 
-    def __init__(self, buffer: torch.Tensor, metadata):
+    ``known``: a list whose one entry is the buffer shape and metadata (a copy)
+    last found to agree, so that a training step does not check them again."""
+
+    __slots__ = ("_buffer", "_metadata", "_known", "_named")
+
+    def __init__(self, buffer: torch.Tensor, metadata, known: list):
         self._buffer = buffer
         self._metadata = metadata
+        self._known = known
+        self._named = None
 
     # Built where a view is asked for: a training step's fused paths need the
     # offsets alone (96 views take 0.18 ms of host time).
-    @cached_property
+    @property
     def _views(self) -> dict[str, torch.Tensor]:
-        return consolidated_dict_view(self._buffer, self._metadata)
+        if self._named is None:
+            self._named = consolidated_dict_view(self._buffer, self._metadata)
+        return self._named
 
     def keys(self):
         return self._views.keys()
@@ -125,26 +130,33 @@ class _GradScatter:
     def __getitem__(self, k):
         return self._views[k]
 
+    def _agrees(self) -> bool:
+        """Whether every parameter's width is its shape's, as the views need."""
+        rows = math.prod(self._buffer.shape[:-1])
+        if any(math.prod(shape) != rows * n for _, shape, _, n in self._metadata):
+            return False
+        if all(type(m) is tuple and isinstance(m[1], tuple) for m in self._metadata):
+            self._known[0] = (self._buffer.shape, list(self._metadata))
+        return True
+
     def segments(self, grads: dict[str, torch.Tensor]):
         """``(tensors, cols)`` for the fused scatter, or None when some
         gradient needs the per-name path (unknown name, other shape, dtype or
         device) or the metadata contradicts itself (the views refuse it)."""
         if type(grads) is not dict:  # any mapping with items()
             grads = dict(grads.items())
-        buf = self._buffer
+        buf, metadata = self._buffer, self._metadata
+        if self._known[0] != (buf.shape, metadata) and not self._agrees():
+            return None
         dtype, device = buf.dtype, buf.device
-        rows = buf.shape[0] if buf.ndim == 2 else math.prod(buf.shape[:-1])
         # A dual tensor carries its tangent without requires_grad.
         tracked = forward_ad._current_level >= 0
         tensors, cols = [], []
-        for name, shape, off, n in self._metadata:  # shape: the stacked (N, *shape)
-            g = grads.get(name, _ABSENT)
-            if g is _ABSENT:
-                if math.prod(shape) != rows * n:
-                    return None
+        for name, shape, off, _ in metadata:  # shape: the stacked (N, *shape)
+            if name not in grads:
                 continue
+            g = grads[name]
             if (not isinstance(g, torch.Tensor) or g.dtype != dtype or g.device != device
-                    or g.numel() != rows * n
                     or (g.shape != shape and tuple(g.shape) != tuple(shape))):
                 return None
             tensors.append(g.detach() if tracked or g.requires_grad else g)
@@ -194,6 +206,7 @@ class State:
         self.active_mask = (active_mask if active_mask is not None
                             else torch.ones(self.batch_size, dtype=torch.bool, device=self.device))
         self.grads = grads if grads is not None else torch.zeros_like(params)
+        self._known_meta: list = [None]
 
     @classmethod
     def from_models(cls, modules: Sequence[Module]) -> "State":
@@ -224,7 +237,7 @@ class State:
 
     @property
     def _consolidated_grads(self) -> _GradScatter:
-        return _GradScatter(self.grads, self.param_meta)
+        return _GradScatter(self.grads, self.param_meta, self._known_meta)
 
     # -- optimizer state ---------------------------------------------------
     def add_optim_state(self, key: str, value: Any = None, per_param: bool = False,

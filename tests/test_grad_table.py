@@ -151,3 +151,26 @@ def test_metadata_that_contradicts_itself_is_refused(bad, given):
     with pytest.raises(RuntimeError):
         SGD.apply_gradient(state, grads)
     assert torch.equal(state.params, before) and not state.grads.any()
+
+
+@pytest.mark.parametrize("meta_type", [torch.Size, list])
+def test_metadata_changed_after_a_step_is_noticed(meta_type):
+    """What was found to agree once is compared by content, not by identity."""
+    state = make(meta_type)
+    grads = grads_of()
+    SGD.apply_gradient(state, grads)
+    good = state.param_meta[0]
+    if meta_type is list:
+        good[1][2] = 1  # the list inside the entry
+    else:
+        state.param_meta[0] = (good[0], good[1], good[2], 5)
+    with pytest.raises(RuntimeError):
+        SGD.apply_gradient(state, grads)
+    if meta_type is list:
+        good[1][2] = 2
+    else:
+        state.param_meta[0] = good
+    SGD.apply_gradient(state, grads)
+    state.grads = state.grads[:3].clone()  # rows that the metadata does not have
+    with pytest.raises(RuntimeError):
+        SGD.apply_gradient(state, grads)
