@@ -473,7 +473,8 @@ constexpr int64_t small_from(int64_t wide, int64_t narrow) {
 // process, mean over 8 and 24 rows; the policies that are not named here stay
 // level or gain as a single launch.
 //   float32 Adam fused 1.2 / 2 / 4 / 8 GB 0.992 / 0.956 / 0.978 / 0.958 (0.5-0.8
-//     GB 1.006-1.002), with bfloat16 moments 2 / 4 / 8 GB 0.993 / 0.974 / 0.992;
+//     GB 1.006-1.002), with bfloat16 moments 2 / 4 / 8 GB 0.993 / 0.974 / 0.992
+//     (three states in turn level at 1.7-2 GB, 0.984 at 3);
 //   float64 Adam fused 0.8 / 2 / 4 GB 0.986 / 0.974 / 0.962 (0.5 GB 1.004);
 //   16-bit Adam kept 2 / 4 / 8 GB 0.986 / 0.960 / 0.952 bfloat16, 1.004 / 0.988 /
 //     0.973 float16, with amsgrad 0.6 / 0.8 / 1.2 / 2 GB 0.983 / 0.977 / 0.957 /
@@ -738,7 +739,8 @@ struct AdamPolicy {
   static constexpr int64_t kBehindFused =
       std::is_same<T, double>::value                        ? 640 * kMiB
       : kFp32State<T, S>                                    ? (AMSGRAD ? kNever : 1024 * kMiB)
-      : kBf16State<T, S> || std::is_same<T, bf16_t>::value ? 1536 * kMiB
+      : kBf16State<T, S>                                    ? 2048 * kMiB
+      : std::is_same<T, bf16_t>::value                      ? 1536 * kMiB
                                                             : kNever;
   static constexpr int kPreWords = 2;
   struct Rep {
