@@ -957,12 +957,10 @@ struct AdagradPolicy {
   // 19-97 MB).
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 1, 1);
   static constexpr bool kScalarMaskSmall = sizeof(T) == 2;
-  // float16 keeps plain accesses up to the MALL's size: from 110 to 240 MB they
-  // are 15-20% ahead with one state resident (110 / 160 / 240 MB 33.3 / 46.1 /
-  // 68.0 us against 40.2 / 55.1 / 79.2) and 4-10% with three in turn (38.7 / 54.9
-  // / 78.7 against 42.7 / 57.9 / 82.3).
+  // 16-bit parameters keep plain accesses up to the MALL's size: the fp64 update
+  // bounds the large shape before the memory does.
   static constexpr int64_t kStreamSmallTo =
-      std::is_same<T, _Float16>::value ? int64_t(256) << 20 : kMallBytes;
+      sizeof(T) == 2 ? int64_t(256) << 20 : kMallBytes;
   static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
   static constexpr int kStreamPack = stream_pack<T, S>();
   // Segmented float32 updates with a workspace: one-wavefront workgroups, one
