@@ -444,13 +444,18 @@ constexpr int64_t kCapMinElems = int64_t(8192) * 512;
 // (so three times the operands pass between two steps of one), plain against
 // non-temporal, same process: float32 Adam at 34 / 51 / 85 / 102 / 119 / 136 /
 // 238 MB 11.9 / 16.1 / 25.3 / 31.1 / 39.9 / 47.9 / 80.3 us against 12.9 / 17.4 /
-// 26.5 / 30.4 / 34.7 / 39.2 / 65.9, and every other optimizer and type but float16
-// Adagrad crosses between 84 and 131 MB too. With one state alone, and nothing
-// else through the cache between its steps, plain accesses stay ahead to the
-// MALL's size: by 0-4% from 130 to 240 MB in float32 Adam and SGD, 4-9% in 16-bit
-// Adam (bfloat16 Adagrad 5-10%; 16-bit SGD loses there too), against the 10-30%
-// that they lose on three states. A training step's activations and gradients
-// pass through the cache, so the line follows the second.
+// 26.5 / 30.4 / 34.7 / 39.2 / 65.9, and every other optimizer and type but 16-bit
+// Adagrad crosses between 84 and 131 MB too. What the line costs the others:
+//   One state alone, with nothing else through the cache between its steps: plain
+//   accesses stay ahead to the MALL's size, at 130-240 MB by 0-5% in 32 and 64
+//   bits and 4-6% in 16-bit Adam (16-bit SGD loses there too), against the 10-30%
+//   that they lose on three states. A training step's activations and gradients
+//   pass through the cache, so the line follows the second.
+//   Three quarters of the rows frozen (the host does not know the mask): the many
+//   short workgroups of the large shape, most of which only leave, bound it, with
+//   plain accesses as well: float32 SGD 11-19 us -> 14-26, without momentum 10-19
+//   -> 15-31, float32 Adagrad +4% to -25%, Adam +20% to -16%, bfloat16 +13% to -2%.
+//   With a quarter frozen the line holds from about 105 MB.
 constexpr int64_t kMallBytes = int64_t(100) << 20;
 
 // The smallest launches of some policies take the large shape too
@@ -958,7 +963,10 @@ struct AdagradPolicy {
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 1, 1);
   static constexpr bool kScalarMaskSmall = sizeof(T) == 2;
   // 16-bit parameters keep plain accesses up to the MALL's size: the fp64 update
-  // bounds the large shape before the memory does.
+  // bounds the large shape before the memory does. Small against large shape at
+  // 110-240 MB, float16 / bfloat16: one state resident +15-20% / +8-13%, three in
+  // turn +3-13% / -3% to +9%, three with a quarter of the rows frozen +4-13% / -4%
+  // to +14%.
   static constexpr int64_t kStreamSmallTo =
       sizeof(T) == 2 ? int64_t(256) << 20 : kMallBytes;
   static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
