@@ -453,8 +453,9 @@ constexpr int64_t kCapMinElems = int64_t(8192) * 512;
 //   pass through the cache, so the line follows the second.
 //   Three quarters of the rows frozen (the host does not know the mask): the many
 //   short workgroups of the large shape, most of which only leave, bound it, with
-//   plain accesses as well: float32 SGD 11-19 us -> 14-26, without momentum 10-19
-//   -> 15-31, float32 Adagrad +4% to -25%, Adam +20% to -16%, bfloat16 +13% to -2%.
+//   plain accesses as well: float32 Adagrad +4% to -25%, Adam +20% to -16%,
+//   bfloat16 +13% to -2%; float32 SGD keeps the small tile there
+//   (kStreamSmallNtTo).
 //   With a quarter frozen the line holds from about 105 MB.
 constexpr int64_t kMallBytes = int64_t(100) << 20;
 
@@ -706,6 +707,7 @@ struct AdamPolicy {
   static constexpr bool kScalarMaskSmall =
       !kFp32State<T, S> && !std::is_same<T, double>::value;
   static constexpr int64_t kStreamSmallTo = kMallBytes;
+  static constexpr int64_t kStreamSmallNtTo = 0;
   static constexpr int64_t kStreamSmallFrom =
       std::is_same<T, bf16_t>::value ? int64_t(48) << 20 : int64_t(28) << 20;
   static constexpr int kStreamPack = stream_pack<T, S>();
@@ -864,6 +866,14 @@ struct SgdPolicy {
   // 128 (same-process A/B, 10 rounds).
   static constexpr int kStreamBlockSmall = kFp32State<T, S> ? 256 : kStreamThreads;
   static constexpr int64_t kStreamSmallTo = kMallBytes;
+  // Float32 state from there to the MALL's size: the small tile with
+  // non-temporal accesses. The large shape's one-wavefront workgroups are four
+  // times as many, and with most rows frozen they are what such a launch waits
+  // for: three quarters frozen, 110 / 160 / 200 / 240 MB 13.2 / 17.1 / 23.5 / 25.6
+  // -> 11.1 / 14.0 / 17.6 / 19.5 us, without momentum 13.9 / 20.6 / 24.4 / 29.5 ->
+  // 9.6 / 13.7 / 16.6 / 19.3; all active +3% to -2%, without momentum -2% to -4%.
+  static constexpr int64_t kStreamSmallNtTo =
+      kFp32State<T, S> ? int64_t(256) << 20 : 0;
   static constexpr int64_t kStreamSmallFrom =
       small_from<T>(std::is_same<T, double>::value ? 16 : 0, 48);
   static constexpr int kStreamPack = stream_pack<T, S>();
@@ -969,6 +979,7 @@ struct AdagradPolicy {
   // to +14%.
   static constexpr int64_t kStreamSmallTo =
       sizeof(T) == 2 ? int64_t(256) << 20 : kMallBytes;
+  static constexpr int64_t kStreamSmallNtTo = 0;
   static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
   static constexpr int kStreamPack = stream_pack<T, S>();
   // Segmented float32 updates with a workspace: one-wavefront workgroups, one
@@ -1102,6 +1113,7 @@ struct AdagradF32Policy {
   // float32: one pack in a single launch (two: -1% to -17% at 19-97 MB).
   static constexpr int kStreamUnrollSmall = stream_unroll<T, S>(1, 1, 4, 1);
   static constexpr int64_t kStreamSmallTo = kMallBytes;
+  static constexpr int64_t kStreamSmallNtTo = 0;
   static constexpr int64_t kStreamSmallFrom = kBf16State<T, S> ? 0 : small_from<T>(16, 0);
   static constexpr int kStreamPack = stream_pack<T, S>();
   // Segmented with a workspace: one-wavefront workgroups, one pack, the
@@ -1777,9 +1789,9 @@ __device__ __forceinline__ void with_maximize(bool maximize, F&& f) {
 // ---------------------------------------------------------------------------
 // FORM: where the per-replica constants come from. A thread's loads are issued
 // before the replica's prologue, which then runs while they are in flight.
-// SMALL: the launch's operands fit the MALL; plain accesses and the small-launch
-// tile instead of non-temporal ones.
-template <typename P, bool ANY, int FORM, bool SMALL>
+// SMALL: the small-launch tile, uncapped, with plain accesses where the launch's
+// operands fit the MALL (NT: non-temporal all the same, kStreamSmallNtTo).
+template <typename P, bool ANY, int FORM, bool SMALL, bool NT = !SMALL>
 __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KArgs<P> a) {
   constexpr bool PRE = pre_of<P, FORM>();
   constexpr bool SINGLE = FORM == kSingle;
@@ -1788,7 +1800,6 @@ __global__ __launch_bounds__((stream_threads<P, SMALL>())) void stream_kernel(KA
   using S = typename P::S;
   constexpr int NS = P::NS;
   constexpr int SS = state_slots<P>();
-  constexpr bool NT = !SMALL;
   constexpr int KP = P::kStreamPack;
   constexpr int U = stream_unroll_of<P, PRE, SMALL>();
   constexpr int64_t kStreamTile = stream_tile<P, PRE, SMALL>();
@@ -3065,17 +3076,17 @@ void launch_column(const ColArgs<P>& ca, uint32_t blocks, bool private_lines,
 
 // The streaming driver over `blocks` tiles, capped when the launch is large
 // (`mid`: the operands take at most kMidBytes; with a workspace only).
-template <typename P, int FORM, bool SMALL>
+template <typename P, int FORM, bool SMALL, bool NT = !SMALL>
 int launch_stream(const KArgs<P>& a, uint32_t blocks, bool same_phase, hipStream_t stream,
                   bool mid) {
   constexpr bool PRE = pre_of<P, FORM>();
   const uint32_t cap = PRE && !SMALL && mid ? P::kStreamLdsMid : stream_lds_of<P, PRE, SMALL>();
   const uint32_t lds = int64_t(blocks) * stream_tile<P, PRE, SMALL>() >= kCapMinElems ? cap : 0u;
   if (same_phase) {
-    hipLaunchKernelGGL((stream_kernel<P, false, FORM, SMALL>), dim3(blocks),
+    hipLaunchKernelGGL((stream_kernel<P, false, FORM, SMALL, NT>), dim3(blocks),
                        dim3(stream_threads<P, SMALL>()), lds, stream, a);
   } else {
-    hipLaunchKernelGGL((stream_kernel<P, true, FORM, SMALL>), dim3(blocks),
+    hipLaunchKernelGGL((stream_kernel<P, true, FORM, SMALL, NT>), dim3(blocks),
                        dim3(stream_threads<P, SMALL>()), lds, stream, a);
   }
   return static_cast<int>(hipGetLastError());
@@ -3095,16 +3106,21 @@ int launch_dense(const Call& c, int nbufs) {
       c.R * c.T * operand_bytes_per_elem<P>() >= P::kStreamSmallFrom;
   const bool mid =
       c.R <= kMidBytes / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1);
+  const int64_t operand_bytes = c.R * c.T * operand_bytes_per_elem<P>();
+  const bool small_nt = (pre || P::kPreWords == 0) && !small &&
+                        operand_bytes > P::kStreamSmallTo &&
+                        operand_bytes <= P::kStreamSmallNtTo;
+  const bool small_tile = small || small_nt;
   const auto prepare = [&] {
     if (!fill_kargs<P>(c, nbufs, a, false)) return false;
     uint32_t res0 = 0, rmod = 0;
     streamable = rows_streamable<P>(a.x, nbufs, res0, rmod);
     const int64_t tile = !streamable ? kElemTile
-                         : small     ? stream_tile<P, false, true>()
+                         : small_tile ? stream_tile<P, false, true>()
                          : pre       ? stream_tile<P, true, false>()
                                      : stream_tile<P, false, false>();
     const int threads = !streamable ? kElemThreads
-                        : small     ? stream_threads<P, true>()
+                        : small_tile ? stream_threads<P, true>()
                                     : stream_threads<P, false>();
     // The streaming driver adds each row's tile 0 (its head and tail).
     if (!make_grid(c.R, c.T, tile, a.g, blocks, threads, streamable)) return false;
@@ -3123,8 +3139,12 @@ int launch_dense(const Call& c, int nbufs) {
     if (streamable) {
       const bool same_phase = rows_same_phase<P>(a.x, nbufs, P::kStreamPack);
       const auto launch = [&](auto form, auto is_small) {
-        return launch_stream<P, decltype(form)::value, decltype(is_small)::value>(
-            a, blocks, same_phase, c.stream, mid);
+        constexpr int F = decltype(form)::value;
+        constexpr bool S = decltype(is_small)::value;
+        if constexpr (!S && P::kStreamSmallNtTo > 0) {
+          if (small_nt) return launch_stream<P, F, true, true>(a, blocks, same_phase, c.stream, mid);
+        }
+        return launch_stream<P, F, S>(a, blocks, same_phase, c.stream, mid);
       };
       // The small shape is built for the forms the operators run: with a
       // workspace where the policy has one, and for SGD, which has none.
