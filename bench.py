@@ -432,18 +432,19 @@ def geometry_timing(rows: int, launches: int, rounds: int = 3):
 # Operand bytes from which a float32 dense launch takes the small shape; below
 # it the policy runs the large launches' (kStreamSmallFrom in optim_drivers.h).
 SMALL_FROM = {"adam": 28 << 20, "sgd": 0, "adagrad": 16 << 20}
-LAUNCH_CLASSES = ("smallest", "small", "mid", "large")
+LAUNCH_CLASSES = ("smallest", "small", "small_nt", "mid", "large")
 
 
 def launch_class(op_name: str, operand_bytes: int) -> str:
     """The launch shape of a float32 dense update over this many bytes of
-    operands: plain accesses and the small shape from SMALL_FROM to 100 MiB, the
-    large shape under a cap of its own up to 1 GiB ("mid") and above, and
-    uncapped below the small one."""
+    operands: plain accesses and the small shape from SMALL_FROM to 100 MiB, for
+    SGD that shape with non-temporal accesses up to 256 MiB, the large shape under
+    a cap of its own up to 1 GiB ("mid") and above, and uncapped below the small
+    one."""
     if operand_bytes > 1 << 30:
         return "large"
     if operand_bytes > 100 << 20:
-        return "mid"
+        return "small_nt" if op_name == "sgd" and operand_bytes <= 256 << 20 else "mid"
     return "small" if operand_bytes >= SMALL_FROM[op_name] else "smallest"
 
 
@@ -1170,10 +1171,11 @@ def main():
                   "true" if op_args[2] is not None else "false", str(kw.get("nesterov")).lower()),
               "adagrad": "AdagradPolicy<float, float>"}[op_name]
     # the instantiation the operator launches: ANY = false (State's layout), FORM = 2 (a single
-    # launch), SMALL (operands that the MALL keeps between steps)
+    # launch), SMALL (the small tile) and NT (non-temporal accesses)
     n_rt = sum(t is not None and t.dim() == 2 for t in op_args)
-    small = launch_class(op_name, op_args[0].numel() * 4 * n_rt) == "small"
-    kernel = "stream_kernel<%s, false, 2, %s>" % (policy, str(small).lower())
+    shape = launch_class(op_name, op_args[0].numel() * 4 * n_rt)
+    kernel = "stream_kernel<%s, false, 2, %s, %s>" % (
+        policy, str(shape in ("small", "small_nt")).lower(), str(shape != "small").lower())
     profile_key = f"{op_name}_stream_kernel_cfg{args.config}"
     hypers = host_hypers(op_name, op_args)
     del op_args

@@ -3100,13 +3100,13 @@ int launch_dense(const Call& c, int nbufs) {
   bool streamable = false;
   const bool pre = uses_workspace<P>(c);
   // Operands that fit the MALL (R, T and the types say so, before any launch).
+  const int64_t operand_bytes = c.R * c.T * operand_bytes_per_elem<P>();
   const bool small =
       (pre || P::kPreWords == 0) &&
       c.R <= P::kStreamSmallTo / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1) &&
-      c.R * c.T * operand_bytes_per_elem<P>() >= P::kStreamSmallFrom;
+      operand_bytes >= P::kStreamSmallFrom;
   const bool mid =
       c.R <= kMidBytes / operand_bytes_per_elem<P>() / std::max<int64_t>(c.T, 1);
-  const int64_t operand_bytes = c.R * c.T * operand_bytes_per_elem<P>();
   const bool small_nt = (pre || P::kPreWords == 0) && !small &&
                         operand_bytes > P::kStreamSmallTo &&
                         operand_bytes <= P::kStreamSmallNtTo;
@@ -3126,8 +3126,7 @@ int launch_dense(const Call& c, int nbufs) {
     if (!make_grid(c.R, c.T, tile, a.g, blocks, threads, streamable)) return false;
     a.g.res0 = res0;
     a.g.rmod = rmod;
-    if (streamable && c.R * c.T * operand_bytes_per_elem<P>() < P::kBehindDense &&
-        single_launch(c)) {
+    if (streamable && operand_bytes < P::kBehindDense && single_launch(c)) {
       a.vec.one = single_of<typename P::T>(c, kEarlyBlocks);
     }
     return true;

@@ -67,5 +67,6 @@ def test_launch_classes(op, edge):
     sizes = [edge * mb - 1, edge * mb, 100 * mb, 100 * mb + 1, 1024 * mb, 1024 * mb + 1]
     assert [bench.launch_class(op, n) for n in sizes] == [
         "smallest", "small", "small", "mid", "mid", "large"]
-    assert bench.launch_class("sgd", 1) == "small"
+    assert [bench.launch_class("sgd", n) for n in (1, 100 * mb + 1, 256 * mb, 256 * mb + 1)] == [
+        "small", "small_nt", "small_nt", "mid"]
     assert bench.launch_class("adam", 4 * 265484 * 16) == "smallest"

@@ -96,6 +96,12 @@ def test_dense_sizes(opt, dtype, state, nbytes):
     check(opt, dtype, state, nbytes, segmented=False)
 
 
+@pytest.mark.parametrize("nbytes", [100 * MB, 255 * MB, 257 * MB])
+def test_sgd_sizes_on_the_small_tile(nbytes):
+    check("sgd", torch.float32, torch.float32, nbytes, segmented=False)
+    check("sgd", torch.float32, torch.bfloat16, nbytes, segmented=False)
+
+
 @pytest.mark.parametrize("nbytes", [639 * MB, 641 * MB])
 def test_dense_sizes_in_one_and_two_launches(nbytes):
     check("adagrad", torch.float32, torch.bfloat16, nbytes, segmented=False)
