@@ -871,7 +871,9 @@ struct SgdPolicy {
   // times as many, and with most rows frozen they are what such a launch waits
   // for: three quarters frozen, 110 / 160 / 200 / 240 MB 13.2 / 17.1 / 23.5 / 25.6
   // -> 11.1 / 14.0 / 17.6 / 19.5 us, without momentum 13.9 / 20.6 / 24.4 / 29.5 ->
-  // 9.6 / 13.7 / 16.6 / 19.3; all active +3% to -2%, without momentum -2% to -4%.
+  // 9.6 / 13.7 / 16.6 / 19.3; all active, three states in turn, +3% to -2%, without
+  // momentum -2% to -4%; one state alone at 130 / 160 / 200 / 240 MB -1% / +3% /
+  // -4% / -7%.
   static constexpr int64_t kStreamSmallNtTo =
       kFp32State<T, S> ? int64_t(256) << 20 : 0;
   static constexpr int64_t kStreamSmallFrom =
